@@ -79,21 +79,14 @@ PRECOMPILE = [
 ] + [
     (0, 256, 8, xcap, 0, 8) for xcap in (1024, 4096)
 ] + [
-    (1, wg, 4, xcap, n, 4) for wg in (256, 512) for n, xcap in ((128, 64), (128, 128), (64, 128), (64, 256),
-                                                              (256, 32), (256, 64))
-] + [
-    (1, 256, 4, xcap, 16, rt) for rt in (1, 2, 4) for xcap in (256, 512, 1024)
+    (1, 128 if n < 64 else 256, 4, 0, n, 1) for n in (4, 8, 12, 16, 32, 48, 64, 72, 80, 128, 256, 512)
 ] + [
     (k, 256, 4, xcap, n, 8) for k in (2, 3) for n in (16, 32, 64, 128, 256) for xcap in (256, 512, 1024, 2048)
 ] + [
     (k, 512, 4, xcap, n, 8) for k in (2, 3) for n in (16, 128) for xcap in (512, 1024, 2048)
 ] + [
-    (1, 512, 4, xcap, 16, 1) for xcap in (256, 512, 1024)
-] + [
     # the 256-matrix batch's SpMM members (N = 16, 128-thread workgroups)
     (k, 128, 4, xcap, 16, 8) for k in (2, 3) for xcap in (256, 512, 1024, 2048)
-] + [
-    (1, 128, 4, xcap, 16, rt) for rt in (1, 2, 4, 8) for xcap in (256, 512, 1024)
 ]
 
 

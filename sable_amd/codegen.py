@@ -60,12 +60,12 @@ def _kernel_source(spec):
     kind, wg, unroll, xcap, nrhs, rtmax = spec
     split = 2 if kind == KIND_SPMM_MFMA2 else 3
     body = {KIND_SPMV: "sb_spmv_body<SB_WG, SB_UNROLL, SB_XCAP>(a);",
-            KIND_SPMM_F32: "sb_spmm_f32_body<SB_WG, SB_RTMAX, SB_NRHS, SB_XCAP>(a);",
+            KIND_SPMM_F32: "sb_spmm_f32_body<SB_NRHS, SB_XCAP != 0>(a);",
             KIND_SPMM_MFMA: "sb_spmm_mfma_body<SB_WG, SB_NRHS, SB_XCAP, SB_SPLIT>(a);",
             KIND_SPMM_MFMA2: "sb_spmm_mfma_body<SB_WG, SB_NRHS, SB_XCAP, SB_SPLIT>(a);"}[kind]
     args = "SbSpmvArgs" if kind == KIND_SPMV else "SbSpmmArgs"
     bounds = {KIND_SPMV: "SB_WG, SB_SPMV_WAVES(SB_UNROLL)",
-              KIND_SPMM_F32: "SB_WG, SB_F32_WAVES(SB_NRHS)"}.get(kind, "SB_WG, SB_MFMA_WAVES")
+              KIND_SPMM_F32: "SB_WG, SB_F32_MINWAVES"}.get(kind, "SB_WG, SB_MFMA_WAVES")
     return (f"// kernel specialisation for this matrix (compiled by hipRTC for gfx950)\n"
             f"#define SB_WG {wg}\n#define SB_UNROLL {unroll}\n#define SB_XCAP {xcap}\n"
             f"#define SB_NRHS {nrhs}\n#define SB_RTMAX {rtmax}\n#define SB_SPLIT {split}\n"

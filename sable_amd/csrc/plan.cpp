@@ -427,16 +427,13 @@ int build_host_plan_once(const SableVbr &v, const uint8_t *route, const SablePla
     S.n_rhs = P.n_rhs;
     S.nblocks = v.nblocks;
 
-    // rows per tile bound: SpMV needs hs <= wg (flat stream lanes).  The FP32
-    // SpMM kernel's wide shape takes 4 rows per thread group, (wg / (N/8)) * 4
-    // rows (8 rows per group measured slower: twice the registers and half
-    // the groups busy); its narrow shape at most 8, (wg / (N/4)) * 8 rows and
-    // 64.  MFMA tiles are cut separately: multiples of 16 rows, at most
+    // rows per tile bound: SpMV needs hs <= wg (flat stream lanes).  FP32 SpMM
+    // tiles are cut into independent wavefront tasks, so their height only
+    // says how many tasks share a panel and X rows through one workgroup.
+    // MFMA tiles are cut separately: multiples of 16 rows, at most
     // mfma_max_rows.
     int max_rows = std::min(o.max_seg_rows, o.wg);
-    if (spmm)
-        max_rows = SB_F32_WIDE(o.n_rhs) ? std::min(max_rows, (o.wg / (o.n_rhs / 8)) * SB_F32_WIDE_ROWS)
-                                        : std::min({max_rows, (o.wg / (o.n_rhs / 4)) * 8, 64});
+    if (spmm) max_rows = std::min(o.max_seg_rows, SB_F32_MAX_ROWS(o.n_rhs));
     const int mfma_rows = spmm && o.n_rhs % 16 == 0
                               ? std::max(16, std::min(SB_MFMA_MAX_ROWS(o.n_rhs, o.wg), (o.max_seg_rows / 16) * 16))
                               : 16;
@@ -516,10 +513,8 @@ int build_host_plan_once(const SableVbr &v, const uint8_t *route, const SablePla
                                                                                     [&](int64_t k) { return geo.keeps(k); })
                                                               : 0);
         S.nblocks_mfma += (int64_t)mfma.size();
-        // FP32 SpMM pieces stage their X rows in LDS (SB_SPMM_XS_FLOATS)
-        const int vcap = spmm ? std::max(1, std::min(o.xcap, SB_SPMM_XS_FLOATS / o.n_rhs)) : o.xcap;
-        auto dgroups = group_columns(dense, v, vcap);
-        auto sgroups = group_columns(sparse, v, vcap);
+        auto dgroups = group_columns(dense, v, o.xcap);
+        auto sgroups = group_columns(sparse, v, o.xcap);
         // MFMA columns: with k chunks, groups of at most kper 32-column
         // k-steps, kper = ceil(K / ceil(K / kchunk)) for the block row's K
         // k-steps, so its chunks are even; each group is then one work item
@@ -676,6 +671,7 @@ int build_host_plan_once(const SableVbr &v, const uint8_t *route, const SablePla
             t.sp_map = -1;
             if (!sp.empty()) {
                 if (spmm) {
+                    std::vector<int32_t> gcols;      // X row of the group's columns
                     for (auto &sr : sp) {
                         SbPiece pc{};
                         pc.kind = SB_PIECE_SPARSE;
@@ -685,6 +681,10 @@ int build_host_plan_once(const SableVbr &v, const uint8_t *route, const SablePla
                         P.srowptr.insert(P.srowptr.end(), sr.rp.begin(), sr.rp.end());
                         P.sval.insert(P.sval.end(), sr.val.begin(), sr.val.end());
                         P.sidx.insert(P.sidx.end(), sr.col.begin(), sr.col.end());
+                        gcols.clear();
+                        for (auto &cs : sgroups[sr.group])
+                            for (int32_t c = 0; c < cs.n; ++c) gcols.push_back(cs.gcol + c);
+                        for (uint16_t c : sr.col) P.scol.push_back(gcols[c]);
                         const int64_t tot = (int64_t)sr.val.size();
                         S.sparse_nnz += tot;
                         S.rowptr_entries += hs + 1;
@@ -729,8 +729,9 @@ int build_host_plan_once(const SableVbr &v, const uint8_t *route, const SablePla
         };
         auto vec_segments = [&](double work_v) {
             int64_t nseg = (h + max_rows - 1) / max_rows;
-            const int64_t want = (int64_t)std::ceil(work_v / (double)o.tile_bytes);
-            return cut(std::max<int64_t>(nseg, std::min<int64_t>(want, (h + min_rows - 1) / min_rows)), false);
+            const int64_t want = spmm ? 1 : (int64_t)std::ceil(work_v / (double)o.tile_bytes);
+            // SpMM: whole 16-row fragments of the matrix instructions
+            return cut(std::max<int64_t>(nseg, std::min<int64_t>(want, (h + min_rows - 1) / min_rows)), spmm);
         };
         if (spmm && !mgroups.empty()) {
             // MFMA tiles (first launch): tall, multiples of 16 rows, only the
@@ -822,5 +823,95 @@ int build_host_plan_once(const SableVbr &v, const uint8_t *route, const SablePla
     return SABLE_OK;
 }
 }  // namespace
+
+std::vector<SbTask> f32_tasks(const std::vector<SbTile> &tiles, const std::vector<SbPiece> &pieces,
+                              const std::vector<SbXRange> &xr, const std::vector<double> &tile_cost, int32_t t0, int32_t t1, int32_t n_rhs)
+{
+    struct Item { SbTask t; double cost; };
+    // clocks of a wavefront: 32 per 16 x 16 x 4 product, about 8 per entry
+    // and 64 columns, and a start
+    auto clocks = [&](double w, double ent, int rows, int height, int cols) {
+        const int u = std::min(2, (rows + 15) / 16), c = (cols + 15) / 16;
+        return 2000.0 + 8.0 * w * u * c + 2.0 * ent * rows / std::max(height, 1) * c;
+    };
+    struct Tile { int64_t w = 0; int32_t rounds = 0; double ent = 0; };
+    std::vector<Tile> info(t1 - t0);
+    for (int32_t k = t0; k < t1; ++k) {
+        const SbTile &tl = tiles[k];
+        Tile &ti = info[k - t0];
+        for (int32_t p = tl.piece_begin; p < tl.piece_end; ++p) {
+            if (pieces[p].kind != SB_PIECE_DENSE) continue;
+            ti.w += pieces[p].ncols;
+            int32_t steps = 0;
+            for (int32_t r = pieces[p].xr_begin; r < pieces[p].xr_end; ++r) steps += (xr[r].len + 7) / 8;
+            ti.rounds += (steps + SB_F32_DEPTH - 1) / SB_F32_DEPTH;
+        }
+        // the tile's sparse entries, from its cost estimate
+        ti.ent = std::max(0.0, (tile_cost[k] - 4.0 * tl.nrows * (double)ti.w - 2.0 * tl.nrows * n_rhs) / 6.0);
+    }
+    std::vector<std::vector<Item>> per_tile;
+    std::vector<double> cost;
+    double total = 0;
+    for (int32_t k = t0; k < t1; ++k) {
+        const SbTile &tl = tiles[k];
+        const Tile &ti = info[k - t0];
+        if (tl.y_accum && tl.piece_begin == tl.piece_end) continue;    // adds nothing
+        const int rows = ti.rounds ? tl.nrows : SB_F32_SPARSE_ROWS(n_rhs) * SB_F32_WAVES(n_rhs);
+        const int cols = ti.rounds ? SB_F32_COLS : 4 << SB_F32_SPARSE_LOGL(n_rhs);
+        per_tile.emplace_back();
+        double sum = 0;
+        for (int32_t n0 = 0; n0 < n_rhs;) {
+            // the rest of N in the least fragments that cover it
+            int c = cols;
+            while (ti.rounds && c > 16 && n_rhs - n0 <= c / 2) c /= 2;
+            for (int32_t r0 = 0; r0 < tl.nrows; r0 += rows) {
+                SbTask t{};
+                t.row0 = tl.row0;
+                t.nrows = tl.nrows;
+                t.piece_begin = tl.piece_begin;
+                t.piece_end = tl.piece_end;
+                t.mat = tl.mat;
+                t.r0 = r0;
+                t.n0 = n0;
+                t.rounds = ti.rounds;
+                t.y_accum = tl.y_accum;
+                t.cols = c;
+                double cst = 0;
+                for (int32_t r = r0; r < std::min(r0 + rows, tl.nrows); r += SB_F32_ROWS)
+                    cst += clocks((double)ti.w, ti.ent, std::min(SB_F32_ROWS, tl.nrows - r), tl.nrows, std::min(c, n_rhs - n0));
+                per_tile.back().push_back({t, cst});
+                sum += cst;
+            }
+            n0 += c;
+        }
+        cost.push_back(sum);
+        total += sum;
+    }
+    std::vector<int32_t> order(per_tile.size());
+    std::iota(order.begin(), order.end(), 0);
+    std::stable_sort(order.begin(), order.end(), [&](int32_t x, int32_t y) { return cost[x] > cost[y]; });
+    std::vector<std::vector<Item>> xcd(SB_XCDS);
+    std::vector<double> load(SB_XCDS, 0.0);
+    auto least = [&] { return (int)(std::min_element(load.begin(), load.end()) - load.begin()); };
+    for (int32_t k : order) {
+        // a tile that is a large part of all work is spread over the XCDs
+        const bool spread = cost[k] > total / (4 * SB_XCDS);
+        int x = least();
+        for (const Item &it : per_tile[k]) {
+            if (spread) x = least();
+            xcd[x].push_back(it);
+            load[x] += it.cost;
+        }
+    }
+    size_t len = 0;
+    for (auto &l : xcd) {
+        std::stable_sort(l.begin(), l.end(), [](const Item &x, const Item &y) { return x.cost > y.cost; });
+        len = std::max(len, l.size());
+    }
+    std::vector<SbTask> out(len * SB_XCDS);
+    for (int x = 0; x < SB_XCDS; ++x)
+        for (size_t i = 0; i < xcd[x].size(); ++i) out[i * SB_XCDS + x] = xcd[x][i].t;
+    return out;
+}
 
 }  // namespace sable

@@ -22,6 +22,7 @@ struct HostPlan {
     std::vector<float> sval;
     std::vector<uint16_t> sidx;
     std::vector<int32_t> srowptr;
+    std::vector<int32_t> scol;    // SpMM: X row of every entry of sval
     std::vector<int32_t> xmap;    // SpMV: x column per staged slot (-1 = zero pad)
     std::vector<double> tile_cost;   // estimated bytes per tile (ordering)
     std::vector<int32_t> tile_phase; // 0: SpMM MFMA tile (first launch), 1: the rest
@@ -39,6 +40,14 @@ SablePlanOpts normalize_opts(const SablePlanOpts *in);
 
 // Returns SABLE_OK or an error code with a message in err.
 int validate_vbr(const SableVbr &v, std::string &err);
+
+// The FP32 SpMM kernel's task list for tiles [t0, t1) (SbTask).  The device
+// hands workgroups to its XCDs round robin, so a tile's tasks all take the
+// places of one XCD (their number modulo SB_XCDS): tiles go to the XCD with
+// the least work so far, largest first, and each XCD's tasks run largest
+// first.  Shorter lists are filled up with empty tasks.
+std::vector<SbTask> f32_tasks(const std::vector<SbTile> &tiles, const std::vector<SbPiece> &pieces,
+                              const std::vector<SbXRange> &xr, const std::vector<double> &tile_cost, int32_t t0, int32_t t1, int32_t n_rhs);
 
 // Builds the host plan.  route may be null (all dense).
 int build_host_plan(const SableVbr &v, const uint8_t *route, const SablePlanOpts &o,

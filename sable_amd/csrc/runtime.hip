@@ -41,9 +41,9 @@ extern "C" __global__ void __launch_bounds__(256, SB_SPMV_WAVES(4)) sb_spmv_aot(
     sb_spmv_body<256, 4, 4096>(a);
 }
 
-extern "C" __global__ void __launch_bounds__(256) sb_spmm_f32_aot(SbSpmmArgs a)
+extern "C" __global__ void __launch_bounds__(256, SB_F32_MINWAVES) sb_spmm_f32_aot(SbSpmmArgs a)
 {
-    sb_spmm_f32_body<256, 8, 0, 4096>(a);
+    sb_spmm_f32_body<0, true>(a);
 }
 
 extern "C" __global__ void __launch_bounds__(256, SB_MFMA_WAVES) sb_spmm_mfma_aot(SbSpmmArgs a)
@@ -306,8 +306,8 @@ const char *kStubSpmv =
     "extern \"C\" __global__ void __launch_bounds__(SB_WG, SB_SPMV_WAVES(SB_UNROLL)) sb_spmv_rtc(SbSpmvArgs a)\n"
     "{ sb_spmv_body<SB_WG, SB_UNROLL, SB_XCAP>(a); }\n";
 const char *kStubSpmmF32 =
-    "extern \"C\" __global__ void __launch_bounds__(SB_WG, SB_F32_WAVES(SB_NRHS)) sb_spmm_f32_rtc(SbSpmmArgs a)\n"
-    "{ sb_spmm_f32_body<SB_WG, SB_RTMAX, SB_NRHS, SB_XCAP>(a); }\n";
+    "extern \"C\" __global__ void __launch_bounds__(SB_WG, SB_F32_MINWAVES) sb_spmm_f32_rtc(SbSpmmArgs a)\n"
+    "{ sb_spmm_f32_body<SB_NRHS, SB_XCAP != 0>(a); }\n";
 const char *kStubSpmmMfma =
     "extern \"C\" __global__ void __launch_bounds__(SB_WG, SB_MFMA_WAVES) sb_spmm_mfma_rtc(SbSpmmArgs a)\n"
     "{ sb_spmm_mfma_body<SB_WG, SB_NRHS, SB_XCAP, SB_SPLIT>(a); }\n";
@@ -334,7 +334,11 @@ struct Phase {
     hipFunction_t fn = nullptr;
     const void *aot = nullptr;
     int grid = 0;
+    int wg = 256;       // workgroup size
+    int32_t ntasks = 0; // FP32 SpMM: the phase's task list has this many places
     int32_t spec[6] = {0, 0, 0, 0, 0, 0};   // kind, wg, unroll, xcap, nrhs, rtmax
+    bool by_task() const { return spec[0] == 1; }   // FP32 SpMM: one workgroup per task
+    int32_t items() const { return by_task() ? ntasks : t1 - t0; }
 };
 
 struct SablePlan {
@@ -354,6 +358,8 @@ struct SablePlan {
     uint16_t *d_sidx = nullptr;
     int32_t *d_srowptr = nullptr;
     int32_t *d_xmap = nullptr;
+    int32_t *d_scol = nullptr;      // SpMM: X row of every sparse entry
+    SbTask *d_tasks = nullptr;      // SpMM: the FP32 kernel's task list
     int32_t *d_queue = nullptr;
     // MFMA tiles split along k: partial-sum scratch and the fixup list
     float *d_part = nullptr;
@@ -380,6 +386,7 @@ struct GroupPart {
     SbTile *d_tiles = nullptr;
     SbPiece *d_pieces = nullptr;
     SbXRange *d_xr = nullptr;
+    SbTask *d_tasks = nullptr;
     SbMatBufs *d_mats = nullptr;
     int32_t *d_queue = nullptr;
     SbTile *d_fix_tiles = nullptr;   // the members' split MFMA row tiles (matrix slot in .mat)
@@ -405,7 +412,9 @@ int upload(T **dptr, const std::vector<T> &v, int64_t &bytes)
 {
     *dptr = nullptr;
     if (v.empty()) return SABLE_OK;
-    HIPOK(hipMalloc((void **)dptr, v.size() * sizeof(T)));
+    // 256 bytes past the end: kernels read one entry past an array's last
+    // (an empty row's first entry) without using it
+    HIPOK(hipMalloc((void **)dptr, v.size() * sizeof(T) + 256));
     HIPOK(hipMemcpy(*dptr, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice));
     bytes += (int64_t)(v.size() * sizeof(T));
     return SABLE_OK;
@@ -435,10 +444,9 @@ int select_phase(const sable::HostPlan &h, const SablePlanOpts &o, Phase &ph)
     s.unroll = o.unroll;
     const bool spmm = h.op == SABLE_OP_SPMM;
     bool mfma = false;
-    int maxcols = 1, maxstage = 1, rows = 1;
+    int maxcols = 1, maxstage = 1;
     for (int32_t t = ph.t0; t < ph.t1; ++t) {
         const SbTile &tl = h.tiles[t];
-        rows = std::max(rows, tl.nrows);
         for (int32_t k = tl.piece_begin; k < tl.piece_end; ++k) {
             const SbPiece &pc = h.pieces[k];
             maxcols = std::max(maxcols, pc.ncols);
@@ -448,25 +456,24 @@ int select_phase(const sable::HostPlan &h, const SablePlanOpts &o, Phase &ph)
     }
     // SpMV: room for the largest staging group the host formed (at most
     // SB_STAGE_CAP + 4 slots, so the buffer never exceeds 4096 + 4)
-    // SpMM: the widest piece's staged columns (the MFMA kernel's k-steps
-    // read up to 31 past them in its padded xrow; the FP32 kernel's X
-    // staging buffer is sized by it, so narrower pieces use less LDS)
-    s.xcap = spmm ? std::min(4096, pow2_at_least(mfma ? maxcols + 1 : maxcols))
+    // MFMA: the widest piece's staged columns (the kernel's k-steps read up
+    // to 31 past them in its padded xrow).  The FP32 kernel stages nothing
+    // there; 1 marks an X of 4 GiB or more, whose rows take 64-bit offsets.
+    const bool far = (int64_t)h.ncols * h.n_rhs * 4 > INT64_C(0xffffffff);
+    s.xcap = spmm ? (mfma ? std::min(4096, pow2_at_least(maxcols + 1)) : (int)far)
                   : std::min(sable::SB_STAGE_CAP, std::max(16, pow2_at_least(maxstage)));
     s.split = o.mfma_split == 2 ? 2 : 3;
     if (spmm) {
         s.nrhs = h.n_rhs;
-        // FP32 kernel: rows per thread group (the wide shape's are whole row quads)
-        const bool wide = SB_F32_WIDE(h.n_rhs);
-        const int ngroups = std::max(1, o.wg / (h.n_rhs / SB_F32_COLS(h.n_rhs)));
-        const int rt = std::max(1, (rows + ngroups - 1) / ngroups);
-        s.rtmax = mfma ? 8 : wide ? (rt + 3) / 4 * 4 : rt;
+        s.rtmax = mfma ? 8 : 1;
+        if (!mfma) s.unroll = 4, s.split = 3, s.wg = SB_F32_WG(h.n_rhs);   // the same kernel whatever these options
     }
     if (spmm)
         ph.aot = mfma ? (s.split == 2 ? (const void *)sb_spmm_mfma2_aot : (const void *)sb_spmm_mfma_aot)
                       : (const void *)sb_spmm_f32_aot;
     else ph.aot = (const void *)sb_spmv_aot;
     ph.spec[0] = spmm ? (mfma ? (s.split == 2 ? 3 : 2) : 1) : 0;
+    ph.wg = s.wg;
     ph.spec[1] = s.wg;
     ph.spec[2] = s.unroll;
     ph.spec[3] = s.xcap;
@@ -512,6 +519,19 @@ int select_phases(const sable::HostPlan &h, const SablePlanOpts &o, int32_t ntil
     return SABLE_OK;
 }
 
+// The task list of the FP32 SpMM phase, if there is one.
+int upload_tasks(const sable::HostPlan &h, std::vector<Phase> &phases, SbTask **d_tasks, int64_t &bytes)
+{
+    for (auto &ph : phases) {
+        if (!ph.by_task()) continue;
+        const std::vector<SbTask> tasks = sable::f32_tasks(h.tiles, h.pieces, h.xr, h.tile_cost, ph.t0, ph.t1, h.n_rhs);
+        if (tasks.size() > (size_t)INT32_MAX) return fail(SABLE_ERR_UNSUPPORTED, "the task list exceeds 2^31 entries");
+        ph.ntasks = (int32_t)tasks.size();
+        CHECKRC(upload(d_tasks, tasks, bytes));
+    }
+    return SABLE_OK;
+}
+
 int occupancy_grid(bool rtc, hipFunction_t fn, const void *aot, int wg, int ntiles, int req)
 {
     if (req > 0) return std::max(1, std::min(req, ntiles));
@@ -548,13 +568,13 @@ int launch_raw(bool rtc, hipFunction_t fn, const void *aot, int grid, int wg, vo
 }
 
 // Launches one phase; events (when given) time this launch alone.
-int launch_phase(int op, int n_rhs, const Phase &ph, int wg, int mode, const SbTile *tiles,
+int launch_phase(int op, int n_rhs, const Phase &ph, int mode, const SbTile *tiles,
                  const SbPiece *pieces, const SbXRange *xr, const float *dval, const float *sval,
-                 const uint16_t *sidx, const int32_t *srowptr, const int32_t *xmap, int32_t *queue,
+                 const uint16_t *sidx, const int32_t *srowptr, const int32_t *xmap, const int32_t *scol, const SbTask *tasks, int32_t *queue,
                  const SbMatBufs *mats, const float *x, float *y, float *part, hipStream_t st,
                  hipEvent_t e0, hipEvent_t e1)
 {
-    const int n = ph.t1 - ph.t0;
+    const int n = ph.items();
     if (n <= 0) return SABLE_OK;
     const int grid = mode == SABLE_MODE_GRID ? n : std::min(ph.grid, n);
     if (op == SABLE_OP_SPMV) {
@@ -563,14 +583,15 @@ int launch_phase(int op, int n_rhs, const Phase &ph, int wg, int mode, const SbT
         a.dval = dval; a.sval = sval; a.sidx = sidx; a.srowptr = srowptr; a.xmap = xmap;
         a.mats = mats; a.x0 = x; a.y0 = y; a.queue = queue;
         a.ntiles = n; a.mode = mode;
-        return launch_raw(ph.rtc, ph.fn, ph.aot, grid, wg, &a, st, e0, e1);
+        return launch_raw(ph.rtc, ph.fn, ph.aot, grid, ph.wg, &a, st, e0, e1);
     }
     SbSpmmArgs a{};
     a.tiles = tiles + ph.t0; a.pieces = pieces; a.xr = xr;
     a.dval = dval; a.sval = sval; a.sidx = sidx; a.srowptr = srowptr;
+    a.scol = scol;
     a.mats = mats; a.x0 = x; a.y0 = y; a.queue = queue; a.part = part;
-    a.ntiles = n; a.mode = mode; a.n_rhs = n_rhs;
-    return launch_raw(ph.rtc, ph.fn, ph.aot, grid, wg, &a, st, e0, e1);
+    a.ntiles = n; a.mode = mode; a.n_rhs = n_rhs; a.tasks = tasks;
+    return launch_raw(ph.rtc, ph.fn, ph.aot, grid, ph.wg, &a, st, e0, e1);
 }
 
 // Launches the fixup of a plan's (or group part's) split MFMA tiles:
@@ -597,9 +618,9 @@ int plan_launch_with(SablePlan *p, const float *x, float *y, float *part, hipEve
     if (e0 && !attached) HIPOK(hipEventRecord(e0, p->stream));
     for (size_t i = 0; i < np; ++i) {
         const Phase &ph = p->phases[i];
-        CHECKRC(launch_phase(p->host.op, p->host.n_rhs, ph, p->opts.wg, p->opts.mode, p->d_tiles, p->d_pieces,
-                             p->d_xr, p->d_dval, p->d_sval, p->d_sidx, p->d_srowptr, p->d_xmap, p->d_queue, nullptr,
-                             x, y, part, p->stream, attached ? e0 : nullptr, attached ? e1 : nullptr));
+        CHECKRC(launch_phase(p->host.op, p->host.n_rhs, ph, p->opts.mode, p->d_tiles, p->d_pieces,
+                             p->d_xr, p->d_dval, p->d_sval, p->d_sidx, p->d_srowptr, p->d_xmap, p->d_scol, p->d_tasks,
+                             p->d_queue, nullptr, x, y, part, p->stream, attached ? e0 : nullptr, attached ? e1 : nullptr));
         if (i == 0 && p->stats.ntiles_mfma > 0)
             CHECKRC(launch_fixup(p->d_fix_tiles, p->nfix, p->fix_groups, nullptr, part, y, p->host.n_rhs, p->stream));
     }
@@ -726,6 +747,7 @@ int sable_plan_create(const SableVbr *vbr, const uint8_t *route, const SablePlan
         no_rtc.wg = 256;       // the spec is recorded, nothing is compiled
         select_phases(p->host, no_rtc, p->stats.ntiles_mfma, p->phases);
         for (auto &ph : p->phases) {
+            if (ph.spec[0] == 1) continue;       // the FP32 SpMM kernel takes neither
             ph.spec[1] = o.wg;
             ph.spec[2] = o.unroll;
         }
@@ -744,6 +766,7 @@ int sable_plan_create(const SableVbr *vbr, const uint8_t *route, const SablePlan
     CHECKRC(upload(&p->d_sidx, h.sidx, bytes));
     CHECKRC(upload(&p->d_srowptr, h.srowptr, bytes));
     CHECKRC(upload(&p->d_xmap, h.xmap, bytes));
+    CHECKRC(upload(&p->d_scol, h.scol, bytes));
     HIPOK(hipMalloc((void **)&p->d_queue, 2 * sizeof(int32_t)));
     HIPOK(hipMemset(p->d_queue, 0, 2 * sizeof(int32_t)));
     if (!h.fix_tiles.empty()) {
@@ -756,8 +779,9 @@ int sable_plan_create(const SableVbr *vbr, const uint8_t *route, const SablePlan
     HIPOK(hipStreamCreateWithFlags(&p->stream, hipStreamNonBlocking));
     p->own_stream = true;
     p->stats.rtc_used = 1;
+    CHECKRC(upload_tasks(h, p->phases, &p->d_tasks, bytes));
     for (auto &ph : p->phases) {
-        ph.grid = occupancy_grid(ph.rtc, ph.fn, ph.aot, o.wg, std::max(1, ph.t1 - ph.t0), o.grid);
+        ph.grid = occupancy_grid(ph.rtc, ph.fn, ph.aot, ph.wg, std::max(1, ph.items()), o.grid);
         p->stats.rtc_used = p->stats.rtc_used && ph.rtc;
     }
     p->stats.grid = p->phases.empty() ? 0 : p->phases[0].grid;
@@ -769,6 +793,7 @@ int sable_plan_create(const SableVbr *vbr, const uint8_t *route, const SablePlan
     p->host.sidx = std::vector<uint16_t>();
     p->host.srowptr = std::vector<int32_t>();
     p->host.xmap = std::vector<int32_t>();
+    p->host.scol = std::vector<int32_t>();
     p->keep_host = false;
     *out = p.release();
     return SABLE_OK;
@@ -779,7 +804,7 @@ int sable_plan_destroy(SablePlan *p)
     if (!p) return SABLE_OK;
     if (p->stream) hipStreamSynchronize(p->stream);
     void *bufs[] = {p->d_tiles, p->d_pieces, p->d_xr, p->d_dval, p->d_sval, p->d_sidx, p->d_srowptr, p->d_xmap,
-                    p->d_queue, p->d_part, p->d_fix_tiles, p->d_xtmp, p->d_ytmp, p->d_flush};
+                    p->d_scol, p->d_tasks, p->d_queue, p->d_part, p->d_fix_tiles, p->d_xtmp, p->d_ytmp, p->d_flush};
     for (void *b : bufs)
         if (b) hipFree(b);
     if (p->own_stream && p->stream) hipStreamDestroy(p->stream);
@@ -947,7 +972,7 @@ namespace {
 
 void free_part(GroupPart &q)
 {
-    void *bufs[] = {q.d_tiles, q.d_pieces, q.d_xr, q.d_mats, q.d_queue, q.d_fix_tiles};
+    void *bufs[] = {q.d_tiles, q.d_pieces, q.d_xr, q.d_tasks, q.d_mats, q.d_queue, q.d_fix_tiles};
     for (void *b : bufs)
         if (b) hipFree(b);
     q = GroupPart();
@@ -999,7 +1024,7 @@ int build_part(SablePlan *const *plans, const std::vector<int> &idx, const float
         b.sval = p->d_sval;
         b.sidx = p->d_sidx;
         b.srowptr = p->d_srowptr;
-        b.xmap = p->d_xmap;
+        b.xmap = p->host.op == SABLE_OP_SPMM ? p->d_scol : p->d_xmap;
         b.x = x[idx[m]];
         b.y = y[idx[m]];
         b.part = p->d_part;
@@ -1038,9 +1063,14 @@ int build_part(SablePlan *const *plans, const std::vector<int> &idx, const float
     view.n_rhs = q.n_rhs;
     view.tiles = sorted;
     view.pieces = pieces;
+    view.xr = xr;
+    view.tile_cost.resize(cost.size());
+    for (size_t i = 0; i < order.size(); ++i) view.tile_cost[i] = cost[order[i]];
+    for (int m : idx) view.ncols = std::max(view.ncols, plans[m]->host.ncols);
     CHECKRC(select_phases(view, p0->opts, nm, q.phases));
+    CHECKRC(upload_tasks(view, q.phases, &q.d_tasks, bytes));
     for (auto &ph : q.phases)
-        ph.grid = occupancy_grid(ph.rtc, ph.fn, ph.aot, q.wg, std::max(1, ph.t1 - ph.t0), grid);
+        ph.grid = occupancy_grid(ph.rtc, ph.fn, ph.aot, ph.wg, std::max(1, ph.items()), grid);
     return SABLE_OK;
 }
 
@@ -1048,8 +1078,8 @@ int launch_part(const GroupPart &q, hipStream_t st)
 {
     const bool has_mfma_phase = q.ntiles_mfma > 0;
     for (size_t i = 0; i < q.phases.size(); ++i) {
-        CHECKRC(launch_phase(q.op, q.n_rhs, q.phases[i], q.wg, q.mode, q.d_tiles, q.d_pieces, q.d_xr, nullptr, nullptr,
-                             nullptr, nullptr, nullptr, q.d_queue, q.d_mats, nullptr, nullptr, nullptr, st, nullptr,
+        CHECKRC(launch_phase(q.op, q.n_rhs, q.phases[i], q.mode, q.d_tiles, q.d_pieces, q.d_xr, nullptr, nullptr,
+                             nullptr, nullptr, nullptr, nullptr, q.d_tasks, q.d_queue, q.d_mats, nullptr, nullptr, nullptr, st, nullptr,
                              nullptr));
         if (i == 0 && has_mfma_phase) CHECKRC(launch_fixup(q.d_fix_tiles, q.nfix, q.fix_groups, q.d_mats, nullptr, nullptr, q.n_rhs, st));
     }

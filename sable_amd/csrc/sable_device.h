@@ -63,20 +63,39 @@ struct SbTile {
 #define SB_SPMV_SPAN_ROWS 256
 #define SB_SPMV_SPAN_VALUES 65536
 
-// LDS for the staged X rows of a FP32 SpMM piece (64 KiB): the plan builder
-// gives such a piece at most SB_SPMM_XS_FLOATS / N columns.
-#define SB_SPMM_XS_FLOATS 16384
+// the device hands workgroups to its XCDs round robin
+#define SB_XCDS 8
 
-// FP32 SpMM thread shape.  Wide (N a multiple of 8, at least 64): a thread
-// holds SB_F32_WIDE_ROWS rows (4 or 8) x 8 columns (two float4 column quads,
-// one in each half of N), so a tile has at most (WG / (N/8)) *
-// SB_F32_WIDE_ROWS rows.  Otherwise: up to 8 rows x one float4 column quad,
-// at most (WG / (N/4)) * 8 rows and 64.
-#define SB_F32_WIDE(N) ((N) >= 64 && (N) % 8 == 0)
-#define SB_F32_COLS(N) (SB_F32_WIDE(N) ? 8 : 4)
-#ifndef SB_F32_WIDE_ROWS
-#define SB_F32_WIDE_ROWS 4
-#endif
+// FP32 SpMM.  A tile with dense pieces is cut into workgroups of 64 columns
+// of Y, each wavefront taking 32 of its rows; a tile without, into workgroups
+// whose wavefronts take SB_F32_SPARSE_ROWS rows x 4 << SB_F32_SPARSE_LOGL
+// columns each.
+#define SB_F32_WAVES(N) ((N) >= 64 ? 4 : 2)
+#define SB_F32_WG(N) (64 * SB_F32_WAVES(N))
+#define SB_F32_ROWS 32
+#define SB_F32_COLS 64
+#define SB_F32_SPARSE_LOGL(N) ((N) > 128 ? 6 : (N) > 64 ? 5 : (N) > 32 ? 4 : (N) > 16 ? 3 : 2)
+#define SB_F32_SPARSE_ITERS 2
+#define SB_F32_SPARSE_ROWS(N) (SB_F32_SPARSE_ITERS * (64 >> SB_F32_SPARSE_LOGL(N)))
+// the tallest FP32 SpMM tile
+#define SB_F32_MAX_ROWS(N) (SB_F32_ROWS * SB_F32_WAVES(N))
+// steps (of 8 columns) of loads in flight per wavefront with dense pieces
+#define SB_F32_DEPTH 3
+
+// One task: rows [r0, ..) of a tile and columns [n0, ..) of Y, with what it
+// needs of the tile (so a wavefront reads one descriptor before its pieces).
+struct SbTask {
+    int32_t row0;            // the tile's first row
+    int32_t nrows;           // the tile's rows; 0: nothing to do (filler)
+    int32_t piece_begin;     // the tile's pieces
+    int32_t piece_end;
+    int32_t mat;             // matrix slot
+    int32_t r0;
+    int32_t n0;
+    int32_t rounds;          // rounds of SB_F32_DEPTH steps over the dense pieces; 0: none
+    int32_t y_accum;         // add to the Y rows an MFMA tile wrote before
+    int32_t cols;            // with dense pieces: columns of the workgroup
+};
 
 // SpMM MFMA tiles: a wavefront holds SB_MFMA_UNITS(N) 16-row tiles across
 // all N/16 column tiles (their FP32 accumulators plus the double-buffered A

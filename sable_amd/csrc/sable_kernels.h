@@ -48,6 +48,31 @@ __device__ __forceinline__ const SB_G T *sb_gp(const T *p)
     return (const SB_G T *)p;
 }
 
+// Read-only descriptors through the constant address space: scalar loads.
+#define SB_K __attribute__((address_space(4)))
+template <typename T>
+__device__ __forceinline__ const SB_K T *sb_kp(const T *p)
+{
+    return (const SB_K T *)p;
+}
+// element i of a descriptor table (uniform i): a copy in scalar registers
+template <typename T>
+__device__ __forceinline__ T sb_kload(const T *p, int i)
+{
+    static_assert(sizeof(T) % 8 == 0, "descriptors are whole 8-byte words");
+    const SB_K uint64_t *s = (const SB_K uint64_t *)(p + i);
+    uint64_t w[sizeof(T) / 8];
+#pragma unroll
+    for (unsigned k = 0; k < sizeof(T) / 8; ++k) w[k] = s[k];
+    return __builtin_bit_cast(T, w);
+}
+
+// a compile-time index for generic lambdas
+template <int V>
+struct SbInt {
+    static constexpr int value = V;
+};
+
 #define SB_MODE_GRID 0      // one workgroup per tile
 #define SB_MODE_STATIC 1    // persistent, tile = wg + k * grid
 #define SB_MODE_QUEUE 2     // persistent, atomic work queue (self-resetting)
@@ -60,7 +85,7 @@ struct SbMatBufs {
     const float *sval;
     const uint16_t *sidx;
     const int32_t *srowptr;
-    const int32_t *xmap;          // SpMV only
+    const int32_t *xmap;          // SpMV: the staging map; SpMM: scol
     const float *x;               // x (SpMV) or X [ncols x n_rhs] (SpMM)
     float *y;                     // y (SpMV) or Y [nrows x n_rhs] (SpMM)
     float *part;                  // SpMM: partial sums of the split MFMA tiles
@@ -92,6 +117,7 @@ struct SbSpmmArgs {
     const float *sval;
     const uint16_t *sidx;
     const int32_t *srowptr;
+    const int32_t *scol;          // X row of every sparse entry
     const SbMatBufs *mats;        // per matrix slot (groups), or null: the fields above
     const float *x0;              // single plan: X
     float *y0;                    // single plan: Y
@@ -100,13 +126,14 @@ struct SbSpmmArgs {
     int32_t ntiles;
     int32_t mode;
     int32_t n_rhs;
+    const SbTask *tasks;          // FP32 kernel: its work list (ntiles tasks)
 };
 
 // The arrays a tile reads: its matrix slot's in a group, else the plan's.
 template <typename Args>
 __device__ __forceinline__ SbMatBufs sb_mat_bufs(const Args &a, int mat, const int32_t *xmap)
 {
-    if (a.mats) return a.mats[mat];
+    if (a.mats) return sb_kload(a.mats, mat);
     SbMatBufs b;
     b.dval = a.dval;
     b.sval = a.sval;
@@ -448,15 +475,472 @@ __device__ __forceinline__ void sb_spmv_body(const SbSpmvArgs &a)
 }
 
 // ---------------------------------------------------------------------------
-// SpMM, FP32 on the vector ALUs (the plain path)
+// SpMM, FP32 (dense pieces on the FP32 matrix instructions, sparse pieces on
+// the vector ALUs)
 //
-// Narrow shape (N not SB_F32_WIDE): thread (rg, v): row group rg = tid / NV
-// owns rows rg*rt .. rg*rt+rt-1 of the tile and RHS columns 4v..4v+3 (NV =
-// n_rhs/4).  Dense piece values are read once per (row, column) and
-// broadcast to the NV lanes of a row group.  The wide shape (below) holds 8
-// columns per thread and reads A as float4 row quads.  Both stage a piece's X
-// rows in LDS once per tile and walk sparse rows entry by entry with the same
-// thread mapping.
+// A tile's work is cut into wavefront tasks that share nothing: a task owns
+// up to 32 rows x 64 columns of Y, keeps them in accumulators and streams
+// its operands from memory straight into registers, so there is no LDS and
+// no barrier, and a compute unit is filled with tasks of any mix of tiles.
+// The host's task list keeps the tasks of a tile on one XCD, since they read
+// the same panel and the same X rows through that XCD's L2.
+//
+// Dense pieces: v_mfma_f32_16x16x4_f32, whose lane l holds A[l%16][l/16] and
+// B[l/16][l%16] (products and sums in FP32).  Which 16 rows and columns a
+// fragment holds is free as long as loads and stores agree, so fragment u of
+// U takes rows U*i + u and fragment t of T columns T*j + t (i, j = l%16): a
+// lane's U rows of a panel column are one vector load and its T columns of
+// an X row another, whole cache lines per wavefront, and its results are
+// T-column vectors of Y.  Per 4 columns of A: two vector loads and U*T
+// matrix instructions of 32 cycles each.
+//
+// Bound: the matrix instructions (256 FLOP per clock and CU, 157 TFLOP/s),
+// twice the vector ALUs' rate without packed instructions.  X rows and A
+// come through L1/L2 at 16 and 4 bytes per clock and CU, far below their
+// rates, so the loads only have to be early enough: SB_F32_DEPTH steps.
+
+// entries whose X rows are in flight in a task without dense pieces (4, 8 or 16)
+#ifndef SB_F32_SPARSE_FLIGHT
+#define SB_F32_SPARSE_FLIGHT 8
+#endif
+// waves per SIMD the launch bound asks of the compiler
+#ifndef SB_F32_MINWAVES
+#define SB_F32_MINWAVES 4
+#endif
+
+typedef float sb_f2 __attribute__((ext_vector_type(2)));
+typedef float sb_c4 __attribute__((ext_vector_type(4)));      // accumulator fragment
+
+// V consecutive floats at p (aligned to their size)
+template <int V>
+__device__ __forceinline__ void sb_load_v(const SB_G float *p, float (&o)[V])
+{
+    if constexpr (V == 4) {
+        const sb_f4 v = *reinterpret_cast<const SB_G sb_f4 *>(p);
+        o[0] = v.x; o[1] = v.y; o[2] = v.z; o[3] = v.w;
+    } else if constexpr (V == 2) {
+        const sb_f2 v = *reinterpret_cast<const SB_G sb_f2 *>(p);
+        o[0] = v.x; o[1] = v.y;
+    } else {
+        o[0] = *p;
+    }
+}
+
+// the same from a uniform base and a 32-bit byte offset (scalar-base loads)
+template <int V>
+__device__ __forceinline__ void sb_load_off(const SB_G float *base, uint32_t bytes, float (&o)[V])
+{
+    sb_load_v<V>(reinterpret_cast<const SB_G float *>(reinterpret_cast<const SB_G char *>(base) + bytes), o);
+}
+
+template <int V>
+__device__ __forceinline__ void sb_store_v(SB_G float *p, const float (&o)[V])
+{
+    if constexpr (V == 4) *reinterpret_cast<SB_G sb_f4 *>(p) = sb_f4{o[0], o[1], o[2], o[3]};
+    else if constexpr (V == 2) *reinterpret_cast<SB_G sb_f2 *>(p) = sb_f2{o[0], o[1]};
+    else *p = o[0];
+}
+
+// Lane K of every 16-lane row (BATCH 16) or of every quad (BATCH 4), to all
+// lanes of that row or quad.
+template <int BATCH, int K>
+__device__ __forceinline__ int sb_bcast(int v)
+{
+    if constexpr (BATCH == 16) return __builtin_amdgcn_update_dpp(0, v, 0x150 + K, 0xf, 0xf, true);   // row_newbcast:K
+    else return __builtin_amdgcn_update_dpp(0, v, K * 0x55, 0xf, 0xf, true);                          // quad_perm:[K,K,K,K]
+}
+
+template <int I, int E, typename F>
+__device__ __forceinline__ void sb_static_for(F f)
+{
+    if constexpr (I < E) {
+        f(SbInt<I>{});
+        sb_static_for<I + 1, E>(f);
+    }
+}
+
+// Adds a batch of a row's entries (lane e of the batch holds entry e: value
+// and X row) to the row's V columns at X + co: n entries of this lane's row
+// are valid (n may differ between the rows of a wavefront), most is the
+// largest n, least the smallest.  F entries' X rows are in flight at a time.
+// Where some row has run out, its entries repeat its last one and add
+// nothing (their X is taken as 0, so an infinity there stays out).  FAR: X is
+// 4 GiB or more.
+template <int BATCH, int F, int V, bool FAR>
+__device__ __forceinline__ void sb_f32_entries(const SB_G float *__restrict__ X, int N, uint32_t co, float val, int col,
+                                               int n, int least, int most, float (&acc)[V])
+{
+    const int off = FAR ? col : (int)((uint32_t)col * (uint32_t)N * 4u);
+    sb_static_for<0, BATCH / F>([&](auto bc) {
+        constexpr int b = decltype(bc)::value;
+        if (F * b < most) {
+            float x[F][V];
+            sb_static_for<0, F>([&](auto kc) {
+                constexpr int k = decltype(kc)::value;
+                const int o = sb_bcast<BATCH, F * b + k>(off);
+                if (FAR) sb_load_v<V>(X + ((int64_t)o * N + co), x[k]);
+                else sb_load_off<V>(X, (uint32_t)o + co * 4u, x[k]);
+            });
+            if (F * b + F > least) {
+#pragma unroll
+                for (int k = 0; k < F; ++k)
+#pragma unroll
+                    for (int j = 0; j < V; ++j) x[k][j] = F * b + k < n ? x[k][j] : 0.f;
+            }
+            sb_static_for<0, F>([&](auto kc) {
+                constexpr int k = decltype(kc)::value;
+                const float v = __builtin_bit_cast(float, sb_bcast<BATCH, F * b + k>(__builtin_bit_cast(int, val)));
+#pragma unroll
+                for (int j = 0; j < V; ++j) acc[j] += v * x[k][j];
+            });
+        }
+    });
+}
+
+// the largest and smallest of a value that is the same over every 2^LOGL lanes
+template <int LOGL>
+__device__ __forceinline__ void sb_range_of(int n, int &least, int &most)
+{
+    if constexpr (LOGL >= 4) {
+        least = most = __builtin_amdgcn_readlane(n, 0);
+#pragma unroll
+        for (int l = 1 << LOGL; l < 64; l += 1 << LOGL) {
+            const int v = __builtin_amdgcn_readlane(n, l);
+            least = min(least, v);
+            most = max(most, v);
+        }
+    } else {
+        int a = n, b = n;
+#pragma unroll
+        for (int m = 1 << LOGL; m < 64; m <<= 1) {
+            a = min(a, __shfl_xor(a, m, 64));
+            b = max(b, __shfl_xor(b, m, 64));
+        }
+        least = __builtin_amdgcn_readfirstlane(a);
+        most = __builtin_amdgcn_readfirstlane(b);
+    }
+}
+
+// A task with dense pieces: rows [r0, r0 + 16U) of its tile, columns
+// [n0, n0 + 16T) of Y.
+template <int U, int T, bool FAR>
+__device__ __forceinline__ void sb_f32_task(const SbSpmmArgs &a, const SbTask &tk, const SbMatBufs &mb, int r0, int N)
+{
+    const int lane = threadIdx.x & 63;
+    const int i = lane & 15, g = lane >> 4;
+    const int hs = tk.nrows, n0 = tk.n0;
+    const int pitch = (hs + 3) & ~3;             // every dense piece of the tile
+    const SB_G float *__restrict__ X = sb_gp(mb.x);
+    const SB_K SbPiece *pieces = sb_kp(a.pieces);
+    const SB_K SbXRange *xr = sb_kp(a.xr);
+    // this lane's rows in a panel column and columns in an X row; past the
+    // panel or the right-hand side they repeat the last ones (never stored)
+    const uint32_t ro = min(r0 + U * i, pitch - U);
+    const uint32_t co = min(n0 + T * i, N - T);
+    const uint32_t va = 4u * (g * pitch + ro), vb = 4u * ((uint32_t)g * N + co);
+    sb_c4 acc[U][T];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int t = 0; t < T; ++t) acc[u][t] = sb_c4{0.f, 0.f, 0.f, 0.f};
+
+    // Each dense piece: the walk over its columns, 8 of one X range per step
+    // (two products of 4), loads SB_F32_DEPTH steps ahead of the products.
+    // Vector instructions take the matrix instructions' time (both run on the
+    // FP32 lanes), so a full step has none: its loads are a scalar base plus
+    // this lane's fixed offsets.  At the end of a range the lanes past it
+    // repeat its last column and are zeroed before their products; past the
+    // last range all are, so the loads are unconditional.
+    constexpr int D = SB_F32_DEPTH;
+    int pi = tk.piece_begin;
+    for (; pi < tk.piece_end && pieces[pi].kind == SB_PIECE_DENSE; ++pi) {
+        int r = pieces[pi].xr_begin;
+        const int re = pieces[pi].xr_end;
+        int left = xr[r].len;
+        const SB_G float *pa = sb_gp(mb.dval) + pieces[pi].data_off;
+        const SB_G float *px = X + (int64_t)xr[r].col0 * N;
+        float av[D][2][U], bv[D][2][T];
+        int rem[D];
+        auto fetch = [&](int d) {
+            rem[d] = left;
+            uint32_t oa0 = va, ob0 = vb, oa1 = va + 16u * pitch, ob1 = vb + 16u * N;
+            if (left < 8) {
+                const int g0 = max(min(g, left - 1), 0), g1 = max(min(g + 4, left - 1), 0);
+                oa0 = 4u * (g0 * pitch + ro);
+                ob0 = 4u * ((uint32_t)g0 * N + co);
+                oa1 = 4u * (g1 * pitch + ro);
+                ob1 = 4u * ((uint32_t)g1 * N + co);
+            }
+            // 32-bit offsets of scalar-base loads, not hoisted to 64-bit adds
+            asm volatile("" : "+v"(oa0), "+v"(ob0), "+v"(oa1), "+v"(ob1));
+            sb_load_off<U>(pa, oa0, av[d][0]);
+            sb_load_off<T>(px, ob0, bv[d][0]);
+            sb_load_off<U>(pa, oa1, av[d][1]);
+            sb_load_off<T>(px, ob1, bv[d][1]);
+            if (left > 8) {
+                left -= 8;
+                pa += 8 * pitch;
+                px += (int64_t)8 * N;
+            } else if (r + 1 < re) {
+                ++r;
+                pa += left * pitch;
+                left = xr[r].len;
+                px = X + (int64_t)xr[r].col0 * N;
+            } else {
+                left = 0;
+            }
+        };
+#pragma unroll
+        for (int d = 0; d < D; ++d) fetch(d);
+        // one exit per round of D steps (several would make the compiler wait
+        // for every load in flight at the loop's head): the last round's
+        // steps past the end multiply zeros
+        do {
+#pragma unroll
+            for (int d = 0; d < D; ++d) {
+                if (rem[d] < 8) {
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        const bool ok = g + 4 * h < rem[d];
+#pragma unroll
+                        for (int u = 0; u < U; ++u) av[d][h][u] = ok ? av[d][h][u] : 0.f;
+#pragma unroll
+                        for (int t = 0; t < T; ++t) bv[d][h][t] = ok ? bv[d][h][t] : 0.f;
+                    }
+                }
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+#pragma unroll
+                    for (int u = 0; u < U; ++u)
+#pragma unroll
+                        for (int t = 0; t < T; ++t)
+                            acc[u][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[d][h][u], bv[d][h][t], acc[u][t], 0, 0, 0);
+                fetch(d);
+            }
+            // the workgroup's wavefronts read the same X rows: a barrier per
+            // round (no data passes) keeps them close, so all but the first
+            // read find them in L1
+            __builtin_amdgcn_s_barrier();
+        } while (rem[0] > 0);
+    }
+
+    // Sparse pieces, into the same accumulators: lane (g, i) holds rows
+    // U*(4g + q) + u (q < 4) and T columns of each, so the four 16-lane rows
+    // of the wavefront walk the entries of four Y rows side by side.
+    for (; pi < tk.piece_end; ++pi) {
+        if (pieces[pi].kind != SB_PIECE_SPARSE) continue;
+        const SB_G int32_t *__restrict__ rp = sb_gp(mb.srowptr) + pieces[pi].rowptr_off;
+        const SB_G float *__restrict__ sv = sb_gp(mb.sval) + pieces[pi].data_off;
+        const SB_G int32_t *__restrict__ sc = sb_gp(mb.xmap) + pieces[pi].data_off;
+        int lo[U][4], n[U][4], c0[U][4];
+        float v0[U][4];
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int row = r0 + U * (4 * g + q) + u;
+                lo[u][q] = rp[min(row, hs - 1)];
+                n[u][q] = (row < hs ? rp[min(row, hs - 1) + 1] : lo[u][q]) - lo[u][q];
+            }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int e = lo[u][q] + max(min(i, n[u][q] - 1), 0);
+                v0[u][q] = sv[e];
+                c0[u][q] = sc[e];
+            }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                float s[T];
+#pragma unroll
+                for (int t = 0; t < T; ++t) s[t] = acc[u][t][q];
+                int least, most;
+                sb_range_of<4>(n[u][q], least, most);
+                float v = v0[u][q];
+                int c = n[u][q] > 0 ? c0[u][q] : 0;
+                for (int e0 = 0; e0 < most; e0 += 16) {
+                    if (e0 > 0) {
+                        const int e = lo[u][q] + max(min(e0 + i, n[u][q] - 1), 0);
+                        v = sv[e];
+                        c = n[u][q] > 0 ? sc[e] : 0;
+                    }
+                    sb_f32_entries<16, 4, T, FAR>(X, N, co, v, c, n[u][q] - e0, least - e0, most - e0, s);
+                }
+#pragma unroll
+                for (int t = 0; t < T; ++t) acc[u][t][q] = s[t];
+            }
+    }
+
+    if (n0 + T * i + T > N) return;
+    SB_G float *__restrict__ Y = sb_gp(mb.y) + (int64_t)tk.row0 * N;
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int row = r0 + U * (4 * g + q) + u;
+            if (row >= hs) continue;
+            SB_G float *dst = Y + (int64_t)row * N + co;
+            float o[T], w[T];
+#pragma unroll
+            for (int t = 0; t < T; ++t) o[t] = acc[u][t][q];
+            if (tk.y_accum) {          // the rows' MFMA tile wrote Y in the previous launch
+                sb_load_v<T>(dst, w);
+#pragma unroll
+                for (int t = 0; t < T; ++t) o[t] += w[t];
+            }
+            sb_store_v<T>(dst, o);
+        }
+}
+
+// A task of a tile without dense pieces: 2^LOGL lanes per row, one float4 of
+// X and Y each (the least that cover N, at least 4 and at most 64; column
+// chunk ch beyond that), so the wavefront walks 64 >> LOGL rows side by side
+// and every X row it meets is one contiguous read.  Its SB_F32_SPARSE_ITERS
+// sets of rows are started together: row pointers of all, first entries of
+// all, then the X rows, so three dependent loads are met once per task and
+// not once per row.
+template <int LOGL, bool FAR>
+__device__ __forceinline__ void sb_f32_sparse_task(const SbSpmmArgs &a, const SbTask &tk, const SbMatBufs &mb, int N)
+{
+    constexpr int L = 1 << LOGL, G = 64 >> LOGL, BATCH = L >= 16 ? 16 : 4, IT = SB_F32_SPARSE_ITERS;
+    constexpr int F = L >= 16 ? SB_F32_SPARSE_FLIGHT : 4;
+    const int lane = threadIdx.x & 63;
+    const int q = lane & (BATCH - 1);
+    const int col = tk.n0 + 4 * (lane & (L - 1));
+    const int r0 = tk.r0 + SB_F32_SPARSE_ROWS(N) * __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (r0 >= tk.nrows) return;
+    const uint32_t co = min(col, N - 4);
+    const int hs = tk.nrows;
+    const SB_G float *__restrict__ X = sb_gp(mb.x);
+    SB_G float *__restrict__ Y = sb_gp(mb.y) + (int64_t)tk.row0 * N + co;
+    const SB_K SbPiece *pieces = sb_kp(a.pieces);
+    float s[IT][4];
+#pragma unroll
+    for (int k = 0; k < IT; ++k) s[k][0] = s[k][1] = s[k][2] = s[k][3] = 0.f;
+    for (int pi = tk.piece_begin; pi < tk.piece_end; ++pi) {
+        const SB_G int32_t *__restrict__ rp = sb_gp(mb.srowptr) + pieces[pi].rowptr_off;
+        const SB_G float *__restrict__ sv = sb_gp(mb.sval) + pieces[pi].data_off;
+        const SB_G int32_t *__restrict__ sc = sb_gp(mb.xmap) + pieces[pi].data_off;
+        int lo[IT], n[IT], c0[IT];
+        float v0[IT];
+#pragma unroll
+        for (int k = 0; k < IT; ++k) {
+            const int row = r0 + k * G + (lane >> LOGL), rr = min(row, hs - 1);
+            lo[k] = rp[rr];
+            n[k] = (row < hs ? rp[rr + 1] : lo[k]) - lo[k];
+        }
+#pragma unroll
+        for (int k = 0; k < IT; ++k) {
+            const int e = lo[k] + max(min(q, n[k] - 1), 0);
+            v0[k] = sv[e];
+            c0[k] = sc[e];
+        }
+#pragma unroll
+        for (int k = 0; k < IT; ++k) {
+            int least, most;
+            sb_range_of<LOGL>(n[k], least, most);
+            float v = v0[k];
+            int c = n[k] > 0 ? c0[k] : 0;
+            for (int e0 = 0; e0 < most; e0 += BATCH) {
+                // the next batch's entries, ahead of this one's X rows
+                const int e = lo[k] + max(min(e0 + BATCH + q, n[k] - 1), 0);
+                const float vn = sv[e];
+                const int cn = sc[e];
+                sb_f32_entries<BATCH, F, 4, FAR>(X, N, co, v, c, n[k] - e0, least - e0, most - e0, s[k]);
+                v = vn;
+                c = n[k] > 0 ? cn : 0;
+            }
+        }
+    }
+    if (col >= N) return;
+#pragma unroll
+    for (int k = 0; k < IT; ++k) {
+        const int row = r0 + k * G + (lane >> LOGL);
+        if (row >= hs) continue;
+        SB_G float *dst = Y + (int64_t)row * N;
+        if (tk.y_accum) {              // the row's MFMA tile wrote Y in the previous launch
+            float w[4];
+            sb_load_v<4>(dst, w);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) s[k][j] += w[j];
+        }
+        sb_store_v<4>(dst, s[k]);
+    }
+}
+
+// A task with dense pieces in fragments for its columns: 64, 32 or 16.
+template <int U, int NRHS, bool FAR>
+__device__ __forceinline__ void sb_f32_columns(const SbSpmmArgs &a, const SbTask &tk, const SbMatBufs &mb, int r0, int N)
+{
+    constexpr int rest = NRHS % 64;          // of N past its groups of 64 columns
+    constexpr bool four = NRHS == 0 || NRHS >= 64 || rest > 32;
+    constexpr bool less = NRHS == 0 || (rest > 0 && rest <= 32);
+    if (four && (!less || tk.cols > 32)) sb_f32_task<U, 4, FAR>(a, tk, mb, r0, N);
+    else if ((NRHS == 0 || rest > 16) && (NRHS != 0 || tk.cols > 16)) sb_f32_task<U, 2, FAR>(a, tk, mb, r0, N);
+    else if (less) sb_f32_task<U, 1, FAR>(a, tk, mb, r0, N);
+}
+
+template <int NRHS, bool FAR>
+__device__ __forceinline__ void sb_f32_work(const SbSpmmArgs &a, int v)
+{
+    const int N = NRHS ? NRHS : a.n_rhs;
+    const SbTask tk = sb_kload(a.tasks, v);
+    if (tk.nrows == 0) return;               // filler of the task list
+    const SbMatBufs mb = sb_mat_bufs(a, tk.mat, a.scol);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (tk.rounds > 0) {
+        const int r0 = SB_F32_ROWS * wave;
+        if (tk.nrows - r0 > 16) sb_f32_columns<2, NRHS, FAR>(a, tk, mb, r0, N);
+        else if (tk.nrows > r0) sb_f32_columns<1, NRHS, FAR>(a, tk, mb, r0, N);
+        else for (int k = 0; k < tk.rounds; ++k) __builtin_amdgcn_s_barrier();
+        return;
+    }
+    if (NRHS) {
+        sb_f32_sparse_task<SB_F32_SPARSE_LOGL(NRHS), FAR>(a, tk, mb, N);
+    } else {
+        switch (SB_F32_SPARSE_LOGL(N)) {
+        case 2: sb_f32_sparse_task<2, FAR>(a, tk, mb, N); break;
+        case 3: sb_f32_sparse_task<3, FAR>(a, tk, mb, N); break;
+        case 4: sb_f32_sparse_task<4, FAR>(a, tk, mb, N); break;
+        case 5: sb_f32_sparse_task<5, FAR>(a, tk, mb, N); break;
+        default: sb_f32_sparse_task<6, FAR>(a, tk, mb, N);
+        }
+    }
+}
+
+// One call site for the three launch modes (the work is inlined once, on a
+// scalar item number): sb_for_tiles' order and queue reset.
+template <int NRHS, bool FAR>
+__device__ __forceinline__ void sb_spmm_f32_body(const SbSpmmArgs &a)
+{
+    __shared__ int next_item;
+    const int items = a.ntiles;
+    const int mode = a.mode;
+    int v = blockIdx.x;
+    for (;;) {
+        if (mode == SB_MODE_QUEUE) {
+            if (threadIdx.x == 0) next_item = atomicAdd(&a.queue[0], 1);
+            __syncthreads();
+            v = __builtin_amdgcn_readfirstlane(next_item);
+            __syncthreads();
+        }
+        if (v >= items) break;
+        sb_f32_work<NRHS, FAR>(a, v);
+        if (mode == SB_MODE_GRID) return;
+        v += gridDim.x;
+    }
+    if (mode == SB_MODE_QUEUE && threadIdx.x == 0) {
+        __threadfence();
+        const int done = atomicAdd(&a.queue[1], 1);
+        if (done == (int)gridDim.x - 1) {
+            atomicExch(&a.queue[0], 0);
+            atomicExch(&a.queue[1], 0);
+        }
+    }
+}
 
 // Expands a piece's x ranges into xrow[0..ncols): the X row of every column.
 __device__ __forceinline__ void sb_expand_xrow(const SbXRange *__restrict__ xr, int r0, int r1, int *xrow)
@@ -467,510 +951,5 @@ __device__ __forceinline__ void sb_expand_xrow(const SbXRange *__restrict__ xr, 
         const int col0 = g->col0, len = g->len;
         for (int i = threadIdx.x; i < len; i += blockDim.x) xrow[base + i] = col0 + i;
         base += len;
-    }
-}
-
-// Stages the X rows of a piece (ncols x N floats, row xrow[c] of X for local
-// column c) into xs4[c * N/4 + v], four float4 loads in flight per thread,
-// coalesced along N.
-template <int WG>
-__device__ __forceinline__ void sb_stage_xrows(const SB_G float *__restrict__ X, int N, const int *xrow, int ncols,
-                                               float4 *xs4)
-{
-    const int NV = N >> 2;
-    const int tot = ncols * NV;
-    for (int i0 = 0; i0 < tot; i0 += 4 * WG) {
-        sb_f4 v[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int i = i0 + u * WG + (int)threadIdx.x;
-            const int c = i < tot ? i / NV : 0;
-            const int q = i < tot ? i - c * NV : 0;
-            v[u] = *reinterpret_cast<const SB_G sb_f4 *>(X + (size_t)xrow[c] * N + 4 * q);
-        }
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int i = i0 + u * WG + (int)threadIdx.x;
-            if (i < tot) reinterpret_cast<sb_f4 *>(xs4)[i] = v[u];
-        }
-    }
-}
-
-struct SbVecMap {
-    int rt;       // rows per row group
-    int rbeg;     // first tile row of this thread's group
-    int v;        // float4 column of this thread
-    bool active;
-};
-
-__device__ __forceinline__ SbVecMap sb_vec_map(int hs, int N, int wg)
-{
-    SbVecMap m;
-    const int NV = N >> 2;
-    const int ngroups = wg / NV;
-    m.rt = (hs + ngroups - 1) / ngroups;
-    const int rg = threadIdx.x / NV;
-    m.v = threadIdx.x - rg * NV;
-    m.active = rg < ngroups;
-    m.rbeg = rg * m.rt;
-    return m;
-}
-
-#ifndef SB_SPMM_SPCHUNK
-#define SB_SPMM_SPCHUNK 512
-#endif
-
-__device__ __forceinline__ void sb_fma4(float4 &acc, float a, const float4 &x)
-{
-    acc.x += a * x.x;
-    acc.y += a * x.y;
-    acc.z += a * x.z;
-    acc.w += a * x.w;
-}
-
-// Accumulates one FP32-dense or sparse piece into acc (RTMAX row registers).
-// The piece's X rows are in LDS (xs4, staged once per tile), so every X read
-// is an LDS read.  Dense: columns are processed 4 at a time with every load
-// of the group issued before its FMAs.  Sparse: the piece's entries are
-// staged through LDS (value and local column) in chunks of SB_SPMM_SPCHUNK,
-// then each thread walks its rows' entries.  spv/spx are LDS scratch of
-// SB_SPMM_SPCHUNK entries.
-template <int WG, int RTMAX>
-__device__ __forceinline__ void sb_spmm_vec_piece(const SbMatBufs &a, const SbPiece &pc, int hs, int N,
-                                                  const SbVecMap &m, const float4 *xs4, float4 *acc, float *spv,
-                                                  int *spx)
-{
-    const int NV = N >> 2;
-    if (pc.kind == SB_PIECE_DENSE) {
-        if (!m.active) return;
-        const SB_G float *__restrict__ P = sb_gp(a.dval) + pc.data_off;
-        int c = 0;
-        for (; c + 4 <= pc.ncols; c += 4) {
-            float4 xv[4];
-            float av[4][RTMAX];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                xv[u] = xs4[(c + u) * NV + m.v];
-                const SB_G float *__restrict__ col = P + (size_t)(c + u) * pc.pitch;
-#pragma unroll
-                for (int i = 0; i < RTMAX; ++i) {
-                    const int r = m.rbeg + i;
-                    av[u][i] = (i < m.rt && r < hs) ? col[r] : 0.f;
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-#pragma unroll
-                for (int i = 0; i < RTMAX; ++i) sb_fma4(acc[i], av[u][i], xv[u]);
-        }
-        for (; c < pc.ncols; ++c) {
-            const float4 xv = xs4[c * NV + m.v];
-            const SB_G float *__restrict__ col = P + (size_t)c * pc.pitch;
-#pragma unroll
-            for (int i = 0; i < RTMAX; ++i) {
-                const int r = m.rbeg + i;
-                if (i < m.rt && r < hs) sb_fma4(acc[i], col[r], xv);
-            }
-        }
-        return;
-    }
-    if (pc.kind != SB_PIECE_SPARSE) return;
-    const SB_G int32_t *__restrict__ rp = sb_gp(a.srowptr) + pc.rowptr_off;
-    const SB_G float *__restrict__ sv = sb_gp(a.sval) + pc.data_off;
-    const SB_G uint16_t *__restrict__ si = sb_gp(a.sidx) + pc.data_off;
-    const int nnzp = rp[hs];
-    int rlo[RTMAX], rhi[RTMAX];
-#pragma unroll
-    for (int i = 0; i < RTMAX; ++i) {
-        const int r = m.rbeg + i;
-        const bool ok = m.active && i < m.rt && r < hs;
-        rlo[i] = ok ? rp[r] : 0;
-        rhi[i] = ok ? rp[r + 1] : 0;
-    }
-    for (int e0 = 0; e0 < nnzp; e0 += SB_SPMM_SPCHUNK) {
-        const int n = min(SB_SPMM_SPCHUNK, nnzp - e0);
-        __syncthreads();
-        for (int e = threadIdx.x; e < n; e += WG) {
-            spv[e] = sv[e0 + e];
-            spx[e] = si[e0 + e];
-        }
-        __syncthreads();
-        if (!m.active) continue;
-#pragma unroll
-        for (int i = 0; i < RTMAX; ++i) {
-            const int lo = max(rlo[i], e0) - e0, hi = min(rhi[i], e0 + n) - e0;
-            int e = lo;
-            for (; e + 4 <= hi; e += 4) {
-                float4 xv[4];
-#pragma unroll
-                for (int u = 0; u < 4; ++u)
-                    xv[u] = xs4[spx[e + u] * NV + m.v];
-#pragma unroll
-                for (int u = 0; u < 4; ++u) sb_fma4(acc[i], spv[e + u], xv[u]);
-            }
-            for (; e < hi; ++e)
-                sb_fma4(acc[i], spv[e], xs4[spx[e] * NV + m.v]);
-        }
-    }
-}
-
-template <int WG, int RTMAX, int NRHS>
-__device__ __forceinline__ void sb_spmm_f32_tile(const SbSpmmArgs &a, int t, int *xrow, float4 *xs4, float *spv,
-                                                 int *spx)
-{
-    const int N = NRHS ? NRHS : a.n_rhs;
-    const SbTile tile = a.tiles[t];
-    const int hs = tile.nrows;
-    const SbVecMap m = sb_vec_map(hs, N, WG);
-    const SbMatBufs mb = sb_mat_bufs(a, tile.mat, nullptr);
-    const SB_G float *__restrict__ X = sb_gp(mb.x);
-    SB_G float *__restrict__ Y = sb_gp(mb.y);
-    float4 acc[RTMAX];
-#pragma unroll
-    for (int i = 0; i < RTMAX; ++i) acc[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-
-    for (int pi = tile.piece_begin; pi < tile.piece_end; ++pi) {
-        const SbPiece pc = a.pieces[pi];
-        __syncthreads();
-        sb_expand_xrow(a.xr, pc.xr_begin, pc.xr_end, xrow);
-        __syncthreads();
-        sb_stage_xrows<WG>(X, N, xrow, pc.ncols, xs4);
-        __syncthreads();
-        sb_spmm_vec_piece<WG, RTMAX>(mb, pc, hs, N, m, xs4, acc, spv, spx);
-    }
-    if (m.active) {
-#pragma unroll
-        for (int i = 0; i < RTMAX; ++i) {
-            const int r = m.rbeg + i;
-            if (i < m.rt && r < hs) {
-                SB_G sb_f4 *dst = reinterpret_cast<SB_G sb_f4 *>(Y + (size_t)(tile.row0 + r) * N + 4 * m.v);
-                sb_f4 o = {acc[i].x, acc[i].y, acc[i].z, acc[i].w};
-                if (tile.y_accum) {      // the rows' MFMA tile wrote Y in the previous launch
-                    const sb_f4 w = *dst;
-                    o = sb_f4{w.x + o.x, w.y + o.y, w.z + o.z, w.w + o.w};
-                }
-                *dst = o;
-            }
-        }
-    }
-}
-
-// Wide shape (SB_F32_WIDE(N)): thread (rg, v) of NV8 = N/8 lanes per row
-// group holds rows [rbeg, rbeg + rt) (rt a multiple of 4 in tiles with dense
-// pieces) and the column quads 4v and N/2 + 4v, so the lanes of a row group
-// read consecutive float4s of the staged X row in each half.  A dense
-// column's row quads are float4 loads from the padded panel (pitch: the
-// rows rounded up to 4), requested SB_F32_DEPTH column pairs ahead through a
-// ring of register sets: per column, one vector-memory load and two LDS
-// loads for 32 FMAs at rt = 4.  Only tiles with dense pieces read row quads
-// (nq >= 1 for every active thread there).
-struct SbWideMap {
-    int rt;       // rows per row group (multiple of 4, uniform over the tile)
-    int rbeg;     // first tile row of this thread's group
-    int v;        // lane in the row group
-    int nq;       // row quads of this thread inside the panel
-    bool active;
-};
-
-// quads: rt rounded up to whole row quads (tiles with dense pieces, whose A
-// columns are read as float4 row quads); else rt = ceil(hs / groups)
-__device__ __forceinline__ SbWideMap sb_wide_map(int hs, int N, int wg, bool quads)
-{
-    SbWideMap m;
-    const int NV8 = N >> 3;
-    const int ngroups = wg / NV8;
-    m.rt = (hs + ngroups - 1) / ngroups;
-    if (quads) m.rt = (m.rt + 3) & ~3;
-    const int rg = threadIdx.x / NV8;
-    m.v = threadIdx.x - rg * NV8;
-    m.rbeg = rg * m.rt;
-    m.active = rg < ngroups && m.rbeg < hs;
-    const int pitch = (hs + 3) & ~3;
-    m.nq = m.active ? min(m.rt, pitch - m.rbeg) >> 2 : 0;
-    return m;
-}
-
-// Wide FP32 SpMM tuning: column pairs of A in flight per thread (register
-// sets of the ring), sparse entries per unrolled step, and the waves per
-// SIMD the launch bound asks of the compiler (4: at most 128 VGPRs, two
-// 512-thread workgroups per CU, which the X staging LDS also allows)
-#ifndef SB_F32_DEPTH
-#define SB_F32_DEPTH 4
-#endif
-#ifndef SB_F32_SPUNROLL
-#define SB_F32_SPUNROLL 4
-#endif
-#ifndef SB_F32_SPCHUNK
-#define SB_F32_SPCHUNK 1536
-#endif
-#ifndef SB_F32_MINWAVES
-#define SB_F32_MINWAVES 4
-#endif
-#define SB_F32_WAVES(N) (SB_F32_WIDE(N) ? SB_F32_MINWAVES : 1)
-
-// r[j] += v * x[j] over the thread's 8 columns
-__device__ __forceinline__ void sb_wide_fma1(float (&r)[8], float v, const float4 &x0, const float4 &x1)
-{
-    r[0] += v * x0.x;
-    r[1] += v * x0.y;
-    r[2] += v * x0.z;
-    r[3] += v * x0.w;
-    r[4] += v * x1.x;
-    r[5] += v * x1.y;
-    r[6] += v * x1.z;
-    r[7] += v * x1.w;
-}
-
-// acc[4q + k][j] += a[q][k] * x[j]
-template <int RQ>
-__device__ __forceinline__ void sb_wide_fma(float (&acc)[4 * RQ][8], const sb_f4 (&a)[RQ], const float4 &x0,
-                                            const float4 &x1)
-{
-#pragma unroll
-    for (int q = 0; q < RQ; ++q) {
-#pragma unroll
-        for (int k = 0; k < 4; ++k) sb_wide_fma1(acc[4 * q + k], a[q][k], x0, x1);
-    }
-}
-
-// The thread's row quads of panel column c.  Quads past the panel (only in
-// the last row group) repeat its last quad: their rows are never stored.
-template <int RQ>
-__device__ __forceinline__ void sb_wide_load(const SB_G float *__restrict__ P, int pitch, int c, int nq,
-                                             sb_f4 (&a)[RQ])
-{
-    const SB_G sb_f4 *__restrict__ col = reinterpret_cast<const SB_G sb_f4 *>(P + (size_t)c * pitch);
-#pragma unroll
-    for (int q = 0; q < RQ; ++q) a[q] = col[min(q, nq - 1)];
-}
-
-// One dense piece: acc += panel x staged X rows.
-template <int RQ>
-__device__ __forceinline__ void sb_spmm_wide_dense(const SbMatBufs &a, const SbPiece &pc, int N, const SbWideMap &m,
-                                                   const float4 *xs4, float (&acc)[4 * RQ][8])
-{
-    const int NV = N >> 2, H = N >> 3;
-    {
-        if (!m.active) return;
-        // column pairs through a ring of SB_F32_DEPTH register sets: the
-        // set just consumed is refilled with the pair SB_F32_DEPTH ahead
-        // (clamped to the last column, so always in bounds)
-        constexpr int D = SB_F32_DEPTH;
-        const int n = pc.ncols, pitch = pc.pitch, np = n >> 1;
-        const SB_G float *__restrict__ P = sb_gp(a.dval) + pc.data_off + m.rbeg;
-        sb_f4 buf[D][2][RQ];
-#pragma unroll
-        for (int d = 0; d < D; ++d) {
-            sb_wide_load<RQ>(P, pitch, min(2 * d, n - 1), m.nq, buf[d][0]);
-            sb_wide_load<RQ>(P, pitch, min(2 * d + 1, n - 1), m.nq, buf[d][1]);
-        }
-        int p = 0;
-        for (; p + D <= np; p += D) {
-#pragma unroll
-            for (int d = 0; d < D; ++d) {
-                const int c = 2 * (p + d);
-                const float4 x00 = xs4[c * NV + m.v], x01 = xs4[c * NV + H + m.v];
-                const float4 x10 = xs4[(c + 1) * NV + m.v], x11 = xs4[(c + 1) * NV + H + m.v];
-                sb_wide_fma<RQ>(acc, buf[d][0], x00, x01);
-                sb_wide_fma<RQ>(acc, buf[d][1], x10, x11);
-                sb_wide_load<RQ>(P, pitch, min(c + 2 * D, n - 1), m.nq, buf[d][0]);
-                sb_wide_load<RQ>(P, pitch, min(c + 2 * D + 1, n - 1), m.nq, buf[d][1]);
-                // keep the refill ahead of the next set's FMAs (the
-                // scheduler otherwise sinks it to the end of the loop)
-                __builtin_amdgcn_sched_barrier(0);
-            }
-        }
-        // the last (np - p) < D pairs are in buf[0 ..]
-#pragma unroll
-        for (int d = 0; d < D - 1; ++d) {
-            if (p + d < np) {
-                const int c = 2 * (p + d);
-                sb_wide_fma<RQ>(acc, buf[d][0], xs4[c * NV + m.v], xs4[c * NV + H + m.v]);
-                sb_wide_fma<RQ>(acc, buf[d][1], xs4[(c + 1) * NV + m.v], xs4[(c + 1) * NV + H + m.v]);
-            }
-        }
-        if (n & 1) {    // odd column count: the last column on its own
-            sb_f4 l[RQ];
-            sb_wide_load<RQ>(P, pitch, n - 1, m.nq, l);
-            sb_wide_fma<RQ>(acc, l, xs4[(n - 1) * NV + m.v], xs4[(n - 1) * NV + H + m.v]);
-        }
-        return;
-    }
-}
-
-// One sparse piece (CSR rows of the tile): its entries are staged in LDS in
-// chunks of SPCH (value, local column), then each thread walks its rows'
-// entries, U entries' loads in flight at a time.
-template <int WG, int RQ, int SPCH, int U>
-__device__ __forceinline__ void sb_spmm_wide_sparse(const SbMatBufs &a, const SbPiece &pc, int hs, int N,
-                                                    const SbWideMap &m, const float4 *xs4,
-                                                    float (&acc)[4 * RQ][8], float *spv, int *spx)
-{
-    const int NV = N >> 2, H = N >> 3;
-    const SB_G int32_t *__restrict__ rp = sb_gp(a.srowptr) + pc.rowptr_off;
-    const SB_G float *__restrict__ sv = sb_gp(a.sval) + pc.data_off;
-    const SB_G uint16_t *__restrict__ si = sb_gp(a.sidx) + pc.data_off;
-    const int nnzp = rp[hs];
-    int rlo[4 * RQ], rhi[4 * RQ];
-#pragma unroll
-    for (int i = 0; i < 4 * RQ; ++i) {
-        const int r = m.rbeg + i;
-        const bool ok = m.active && i < m.rt && r < hs;
-        rlo[i] = ok ? rp[r] : 0;
-        rhi[i] = ok ? rp[r + 1] : 0;
-    }
-    for (int e0 = 0; e0 < nnzp; e0 += SPCH) {
-        const int cnt = min(SPCH, nnzp - e0);
-        __syncthreads();
-        for (int e = threadIdx.x; e < cnt; e += WG) {
-            spv[e] = sv[e0 + e];
-            spx[e] = si[e0 + e];
-        }
-        __syncthreads();
-        if (!m.active) continue;
-#pragma unroll
-        for (int i = 0; i < 4 * RQ; ++i) {
-            const int lo = max(rlo[i], e0) - e0, hi = min(rhi[i], e0 + cnt) - e0;
-            // SB_F32_SPUNROLL entries' loads in flight, then their FMAs in
-            // entry order
-            int e = lo;
-            for (; e + U <= hi; e += U) {
-                float v[U];
-                float4 x0[U], x1[U];
-#pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    v[u] = spv[e + u];
-                    const int ci = spx[e + u];
-                    x0[u] = xs4[ci * NV + m.v];
-                    x1[u] = xs4[ci * NV + H + m.v];
-                }
-#pragma unroll
-                for (int u = 0; u < U; ++u) sb_wide_fma1(acc[i], v[u], x0[u], x1[u]);
-            }
-            for (; e < hi; ++e) {
-                const int ci = spx[e];
-                sb_wide_fma1(acc[i], spv[e], xs4[ci * NV + m.v], xs4[ci * NV + H + m.v]);
-            }
-        }
-    }
-}
-
-// Stages the X rows of piece pc into xs4 (after every thread is done with
-// the previous piece's).
-template <int WG>
-__device__ __forceinline__ void sb_wide_stage(const SbSpmmArgs &a, const SbPiece &pc, const SB_G float *X, int N,
-                                              int *xrow, float4 *xs4)
-{
-    __syncthreads();
-    sb_expand_xrow(a.xr, pc.xr_begin, pc.xr_end, xrow);
-    __syncthreads();
-    sb_stage_xrows<WG>(X, N, xrow, pc.ncols, xs4);
-    __syncthreads();
-}
-
-// One tile with up to 4 * RQ rows per thread group: its dense pieces first,
-// then its sparse pieces (two loops, so the registers the dense loop keeps
-// are free in the sparse one).  DENSE false: the tile has no dense pieces.
-template <int WG, int RQ, int NRHS, bool DENSE>
-__device__ __forceinline__ void sb_spmm_wide_tile_q(const SbSpmmArgs &a, const SbTile &tile, const SbWideMap &m,
-                                                    int *xrow, float4 *xs4, float *spv, int *spx)
-{
-    const int N = NRHS ? NRHS : a.n_rhs;
-    const int hs = tile.nrows;
-    const SbMatBufs mb = sb_mat_bufs(a, tile.mat, nullptr);
-    const SB_G float *__restrict__ X = sb_gp(mb.x);
-    SB_G float *__restrict__ Y = sb_gp(mb.y);
-    float acc[4 * RQ][8];
-#pragma unroll
-    for (int i = 0; i < 4 * RQ; ++i)
-#pragma unroll
-        for (int j = 0; j < 8; ++j) acc[i][j] = 0.f;
-
-    if constexpr (DENSE) {
-        for (int pi = tile.piece_begin; pi < tile.piece_end; ++pi) {
-            const SbPiece pc = a.pieces[pi];
-            if (pc.kind != SB_PIECE_DENSE) continue;
-            sb_wide_stage<WG>(a, pc, X, N, xrow, xs4);
-            sb_spmm_wide_dense<RQ>(mb, pc, N, m, xs4, acc);
-        }
-    }
-    for (int pi = tile.piece_begin; pi < tile.piece_end; ++pi) {
-        const SbPiece pc = a.pieces[pi];
-        if (pc.kind != SB_PIECE_SPARSE) continue;
-        sb_wide_stage<WG>(a, pc, X, N, xrow, xs4);
-        sb_spmm_wide_sparse<WG, RQ, SB_F32_SPCHUNK, SB_F32_SPUNROLL>(mb, pc, hs, N, m, xs4, acc, spv, spx);
-    }
-    if (!m.active) return;
-#pragma unroll
-    for (int i = 0; i < 4 * RQ; ++i) {
-        const int r = m.rbeg + i;
-        if (i < m.rt && r < hs) {
-            SB_G float *row = Y + (size_t)(tile.row0 + r) * N + 4 * m.v;
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                SB_G sb_f4 *dst = reinterpret_cast<SB_G sb_f4 *>(row + h * (N >> 1));
-                sb_f4 o = {acc[i][4 * h], acc[i][4 * h + 1], acc[i][4 * h + 2], acc[i][4 * h + 3]};
-                if (tile.y_accum) {      // the rows' MFMA tile wrote Y in the previous launch
-                    const sb_f4 w = *dst;
-                    o = sb_f4{w.x + o.x, w.y + o.y, w.z + o.z, w.w + o.w};
-                }
-                *dst = o;
-            }
-        }
-    }
-}
-
-// rt (uniform over the tile, at most 4 * RQ) picks the instance: 4 or 8
-// rows per thread group, with or without the dense loop.
-template <int WG, int RQ, int NRHS>
-__device__ __forceinline__ void sb_spmm_wide_tile(const SbSpmmArgs &a, int t, int *xrow, float4 *xs4, float *spv,
-                                                  int *spx)
-{
-    static_assert(RQ == 1 || RQ == 2, "the wide shape holds 4 or 8 rows per thread group");
-    const int N = NRHS ? NRHS : a.n_rhs;
-    const SbTile tile = a.tiles[t];
-    bool dense = false;
-    for (int pi = tile.piece_begin; pi < tile.piece_end; ++pi) dense = dense || a.pieces[pi].kind == SB_PIECE_DENSE;
-    const SbWideMap m = sb_wide_map(tile.nrows, N, WG, dense);
-    if (dense) {
-        if (RQ == 2 && m.rt > 4) sb_spmm_wide_tile_q<WG, RQ, NRHS, true>(a, tile, m, xrow, xs4, spv, spx);
-        else sb_spmm_wide_tile_q<WG, 1, NRHS, true>(a, tile, m, xrow, xs4, spv, spx);
-    } else {
-        if (RQ == 2 && m.rt > 4) sb_spmm_wide_tile_q<WG, RQ, NRHS, false>(a, tile, m, xrow, xs4, spv, spx);
-        else sb_spmm_wide_tile_q<WG, 1, NRHS, false>(a, tile, m, xrow, xs4, spv, spx);
-    }
-}
-
-template <int WG, int RTMAX, int NRHS, int XCAP>
-__device__ __forceinline__ void sb_spmm_f32_body(const SbSpmmArgs &a)
-{
-    // staged X rows of the current piece: pieces have at most
-    // SB_SPMM_XS_FLOATS / N columns (the plan builder cuts them so)
-    constexpr int XS4 = NRHS ? (XCAP < SB_SPMM_XS_FLOATS / NRHS ? XCAP : SB_SPMM_XS_FLOATS / NRHS) * (NRHS / 4)
-                             : SB_SPMM_XS_FLOATS / 4;
-    __shared__ int xrow[XCAP + 4];
-    __shared__ float4 xs4[XS4];
-    // sparse entry chunks: SB_F32_SPCHUNK entries in the wide shape,
-    // SB_SPMM_SPCHUNK in the narrow one (the generic instance runs either)
-    constexpr int SPC = NRHS == 0 ? (SB_F32_SPCHUNK > SB_SPMM_SPCHUNK ? SB_F32_SPCHUNK : SB_SPMM_SPCHUNK)
-                        : SB_F32_WIDE(NRHS) ? SB_F32_SPCHUNK : SB_SPMM_SPCHUNK;
-    __shared__ float spv[SPC];
-    __shared__ int spx[SPC];
-    __shared__ int next_tile;
-    // wide: tiles hold at most SB_F32_WIDE_ROWS rows per thread group (the
-    // plan builder cuts them so); RTMAX <= 4 leaves out the 8-row instance
-    constexpr int RQ = RTMAX > 4 ? 2 : 1;
-    if constexpr (NRHS != 0 && SB_F32_WIDE(NRHS)) {
-        sb_for_tiles(a.ntiles, a.mode, a.queue, &next_tile,
-                     [&](int t) { sb_spmm_wide_tile<WG, RQ, NRHS>(a, t, xrow, xs4, spv, spx); });
-    } else if constexpr (NRHS != 0) {
-        sb_for_tiles(a.ntiles, a.mode, a.queue, &next_tile,
-                     [&](int t) { sb_spmm_f32_tile<WG, RTMAX, NRHS>(a, t, xrow, xs4, spv, spx); });
-    } else if (SB_F32_WIDE(a.n_rhs)) {     // generic instance: the shape follows N
-        sb_for_tiles(a.ntiles, a.mode, a.queue, &next_tile,
-                     [&](int t) { sb_spmm_wide_tile<WG, SB_F32_WIDE_ROWS / 4, 0>(a, t, xrow, xs4, spv, spx); });
-    } else {
-        sb_for_tiles(a.ntiles, a.mode, a.queue, &next_tile,
-                     [&](int t) { sb_spmm_f32_tile<WG, RTMAX, NRHS>(a, t, xrow, xs4, spv, spx); });
     }
 }

@@ -191,11 +191,6 @@ __device__ __forceinline__ void sb_store_b(int N, int ncols, int ks, float (*f)[
 // The product passes over the term pairs (a_i, x_j) with i + j < SPLIT,
 // smallest terms first: SPLIT = 3 -> a3x1 a2x2 a1x3 a2x1 a1x2 a1x1,
 // SPLIT = 2 -> a2x1 a1x2 a1x1.
-template <int V>
-struct SbInt {
-    static constexpr int value = V;
-};
-
 template <int SPLIT>
 struct SbPasses {
     static constexpr int N = SPLIT == 3 ? 6 : 3;
