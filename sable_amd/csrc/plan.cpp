@@ -834,6 +834,10 @@ std::vector<SbTask> f32_tasks(const std::vector<SbTile> &tiles, const std::vecto
         const int u = std::min(2, (rows + 15) / 16), c = (cols + 15) / 16;
         return 2000.0 + 8.0 * w * u * c + 2.0 * ent * rows / std::max(height, 1) * c;
     };
+    // rows per wavefront: 32, whose two fragments share every X value; 16 if
+    // that leaves a SIMD fewer than two wavefronts, whose time is then its
+    // chain of loads
+    int64_t waves = 0;
     struct Tile { int64_t w = 0; int32_t rounds = 0; double ent = 0; };
     std::vector<Tile> info(t1 - t0);
     for (int32_t k = t0; k < t1; ++k) {
@@ -846,9 +850,11 @@ std::vector<SbTask> f32_tasks(const std::vector<SbTile> &tiles, const std::vecto
             for (int32_t r = pieces[p].xr_begin; r < pieces[p].xr_end; ++r) steps += (xr[r].len + 7) / 8;
             ti.rounds += (steps + SB_F32_DEPTH - 1) / SB_F32_DEPTH;
         }
+        if (ti.rounds) waves += (int64_t)((tl.nrows + 31) / 32) * ((n_rhs + SB_F32_COLS - 1) / SB_F32_COLS);
         // the tile's sparse entries, from its cost estimate
         ti.ent = std::max(0.0, (tile_cost[k] - 4.0 * tl.nrows * (double)ti.w - 2.0 * tl.nrows * n_rhs) / 6.0);
     }
+    const int wrows = waves < 2 * SB_SIMDS ? 16 : 32;
     std::vector<std::vector<Item>> per_tile;
     std::vector<double> cost;
     double total = 0;
@@ -856,7 +862,7 @@ std::vector<SbTask> f32_tasks(const std::vector<SbTile> &tiles, const std::vecto
         const SbTile &tl = tiles[k];
         const Tile &ti = info[k - t0];
         if (tl.y_accum && tl.piece_begin == tl.piece_end) continue;    // adds nothing
-        const int rows = ti.rounds ? tl.nrows : SB_F32_SPARSE_ROWS(n_rhs) * SB_F32_WAVES(n_rhs);
+        const int rows = ti.rounds ? wrows * SB_F32_WAVES(n_rhs) : SB_F32_SPARSE_ROWS(n_rhs) * SB_F32_WAVES(n_rhs);
         const int cols = ti.rounds ? SB_F32_COLS : 4 << SB_F32_SPARSE_LOGL(n_rhs);
         per_tile.emplace_back();
         double sum = 0;
@@ -875,10 +881,11 @@ std::vector<SbTask> f32_tasks(const std::vector<SbTile> &tiles, const std::vecto
                 t.n0 = n0;
                 t.rounds = ti.rounds;
                 t.y_accum = tl.y_accum;
-                t.cols = c;
+                t.cols = (uint16_t)c;
+                t.rows = (uint16_t)wrows;
                 double cst = 0;
-                for (int32_t r = r0; r < std::min(r0 + rows, tl.nrows); r += SB_F32_ROWS)
-                    cst += clocks((double)ti.w, ti.ent, std::min(SB_F32_ROWS, tl.nrows - r), tl.nrows, std::min(c, n_rhs - n0));
+                for (int32_t r = r0; r < std::min(r0 + rows, tl.nrows); r += wrows)
+                    cst += clocks((double)ti.w, ti.ent, std::min(wrows, tl.nrows - r), tl.nrows, std::min(c, n_rhs - n0));
                 per_tile.back().push_back({t, cst});
                 sum += cst;
             }

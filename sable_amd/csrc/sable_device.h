@@ -65,9 +65,10 @@ struct SbTile {
 
 // the device hands workgroups to its XCDs round robin
 #define SB_XCDS 8
+#define SB_SIMDS 1024
 
 // FP32 SpMM.  A tile with dense pieces is cut into workgroups of 64 columns
-// of Y, each wavefront taking 32 of its rows; a tile without, into workgroups
+// of Y, each wavefront taking 32 (or 16) of its rows; a tile without, into workgroups
 // whose wavefronts take SB_F32_SPARSE_ROWS rows x 4 << SB_F32_SPARSE_LOGL
 // columns each.
 #define SB_F32_WAVES(N) ((N) >= 64 ? 4 : 2)
@@ -94,7 +95,8 @@ struct SbTask {
     int32_t n0;
     int32_t rounds;          // rounds of SB_F32_DEPTH steps over the dense pieces; 0: none
     int32_t y_accum;         // add to the Y rows an MFMA tile wrote before
-    int32_t cols;            // with dense pieces: columns of the workgroup
+    uint16_t cols;           // with dense pieces: columns of the workgroup and
+    uint16_t rows;           // rows of each wavefront (32 or 16)
 };
 
 // SpMM MFMA tiles: a wavefront holds SB_MFMA_UNITS(N) 16-row tiles across

@@ -478,12 +478,10 @@ __device__ __forceinline__ void sb_spmv_body(const SbSpmvArgs &a)
 // SpMM, FP32 (dense pieces on the FP32 matrix instructions, sparse pieces on
 // the vector ALUs)
 //
-// A tile's work is cut into wavefront tasks that share nothing: a task owns
-// up to 32 rows x 64 columns of Y, keeps them in accumulators and streams
-// its operands from memory straight into registers, so there is no LDS and
-// no barrier, and a compute unit is filled with tasks of any mix of tiles.
-// The host's task list keeps the tasks of a tile on one XCD, since they read
-// the same panel and the same X rows through that XCD's L2.
+// A wavefront owns up to 32 rows x 64 columns of Y, keeps them in
+// accumulators and streams its operands from memory into registers; no data
+// goes through LDS.  The host's task list (SbTask) keeps the workgroups of a
+// tile on one XCD, whose L2 then serves the panel and X rows they share.
 //
 // Dense pieces: v_mfma_f32_16x16x4_f32, whose lane l holds A[l%16][l/16] and
 // B[l/16][l%16] (products and sums in FP32).  Which 16 rows and columns a
@@ -492,12 +490,19 @@ __device__ __forceinline__ void sb_spmv_body(const SbSpmvArgs &a)
 // lane's U rows of a panel column are one vector load and its T columns of
 // an X row another, whole cache lines per wavefront, and its results are
 // T-column vectors of Y.  Per 4 columns of A: two vector loads and U*T
-// matrix instructions of 32 cycles each.
+// matrix instructions of 32 clocks each.
 //
 // Bound: the matrix instructions (256 FLOP per clock and CU, 157 TFLOP/s),
-// twice the vector ALUs' rate without packed instructions.  X rows and A
-// come through L1/L2 at 16 and 4 bytes per clock and CU, far below their
-// rates, so the loads only have to be early enough: SB_F32_DEPTH steps.
+// twice the vector ALUs' rate without packed instructions.  The vector
+// kernel this replaced (4 rows x 8 columns per thread, X staged in LDS) took
+// 260 us on the 50,000-row SpMM at N = 128 (35 M dense values, 0.9 M
+// entries) and 122 us on a 3,001-row one at N = 512; this one takes 175 and
+// 34 us.  On dense blocks alone it runs at 69 TFLOP/s (127 us): vector and
+// memory instructions take matrix time (both use the FP32 lanes and register
+// ports), and long tiles share SIMDs with others.  Measured slower, dense
+// blocks alone / with the entries: X staged through LDS (149 / 188 us),
+// 32-column tasks (155 / 213 us), one wavefront per workgroup without the
+// barrier (132 / 184 us).
 
 // entries whose X rows are in flight in a task without dense pieces (4, 8 or 16)
 #ifndef SB_F32_SPARSE_FLIGHT
@@ -892,8 +897,8 @@ __device__ __forceinline__ void sb_f32_work(const SbSpmmArgs &a, int v)
     const SbMatBufs mb = sb_mat_bufs(a, tk.mat, a.scol);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if (tk.rounds > 0) {
-        const int r0 = SB_F32_ROWS * wave;
-        if (tk.nrows - r0 > 16) sb_f32_columns<2, NRHS, FAR>(a, tk, mb, r0, N);
+        const int r0 = tk.r0 + tk.rows * wave;
+        if (tk.rows > 16 && tk.nrows - r0 > 16) sb_f32_columns<2, NRHS, FAR>(a, tk, mb, r0, N);
         else if (tk.nrows > r0) sb_f32_columns<1, NRHS, FAR>(a, tk, mb, r0, N);
         else for (int k = 0; k < tk.rounds; ++k) __builtin_amdgcn_s_barrier();
         return;
