@@ -338,7 +338,13 @@ struct Phase {
     int32_t ntasks = 0; // FP32 SpMM: the phase's task list has this many places
     int32_t spec[6] = {0, 0, 0, 0, 0, 0};   // kind, wg, unroll, xcap, nrhs, rtmax
     bool by_task() const { return spec[0] == 1; }   // FP32 SpMM: one workgroup per task
-    int32_t items() const { return by_task() ? ntasks : t1 - t0; }
+    // workgroups (work items) of the phase; MFMA: one per tile and column
+    // group (the generic kernel takes all columns at once)
+    int32_t items() const
+    {
+        const int32_t groups = spec[0] >= 2 && rtc ? spec[4] / SB_MFMA_COLS(spec[4], wg) : 1;
+        return by_task() ? ntasks : (t1 - t0) * groups;
+    }
 };
 
 struct SablePlan {

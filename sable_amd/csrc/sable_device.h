@@ -99,12 +99,22 @@ struct SbTask {
     uint16_t rows;           // rows of each wavefront (32 or 16)
 };
 
-// SpMM MFMA tiles: a wavefront holds SB_MFMA_UNITS(N) 16-row tiles across
-// all N/16 column tiles (their FP32 accumulators plus the double-buffered A
-// fragments), which bounds a tile at SB_MFMA_MAX_ROWS(N, WG) rows (and 256).
-#define SB_MFMA_UNITS(N) ((N) >= 256 ? 1 : 2)
-#define SB_MFMA_MAX_ROWS(N, WG) \
-    (16 * ((WG) / 64) * SB_MFMA_UNITS(N) < 256 ? 16 * ((WG) / 64) * SB_MFMA_UNITS(N) : 256)
+// SpMM MFMA tiles: a workgroup takes SB_MFMA_COLS(N, WG) columns of Y (N over
+// that many workgroups per tile): up to 64 in workgroups of at most 256
+// threads, whose registers and LDS then leave room for two or three of them
+// on a compute unit, all of N in larger ones.  On the 50,000-row SpMM at
+// N = 128 (dense blocks alone) 64-column workgroups of 256 threads took
+// 88 us and full-width ones 107 us; at 512 threads 100 us and 84 us.
+// A wavefront holds two 16-row units across the columns (their FP32
+// accumulators plus the double-buffered A fragments), which bounds a tile at
+// SB_MFMA_MAX_ROWS(N, WG) rows (and 256).
+#define SB_MFMA_COLS(N, WG)                                                                                 \
+    ((N) <= 64 || (WG) > 256 ? (N) : (N) % 64 == 0 ? 64 : (N) % 48 == 0 ? 48 : (N) % 32 == 0 ? 32 : (N))
+#define SB_MFMA_UNITS(COLS) ((COLS) >= 256 ? 1 : 2)
+#define SB_MFMA_MAX_ROWS(N, WG)                                     \
+    (16 * ((WG) / 64) * SB_MFMA_UNITS(SB_MFMA_COLS(N, WG)) < 256    \
+         ? 16 * ((WG) / 64) * SB_MFMA_UNITS(SB_MFMA_COLS(N, WG))    \
+         : 256)
 
 // A panel piece of a tile: the tile's rows restricted to a group of blocks
 // whose columns (ncols <= the x staging capacity) are staged in LDS.

@@ -133,7 +133,7 @@ struct SbSpmmArgs {
 template <typename Args>
 __device__ __forceinline__ SbMatBufs sb_mat_bufs(const Args &a, int mat, const int32_t *xmap)
 {
-    if (a.mats) return sb_kload(a.mats, mat);
+    if (a.mats) return a.mats[mat];
     SbMatBufs b;
     b.dval = a.dval;
     b.sval = a.sval;
@@ -894,7 +894,7 @@ __device__ __forceinline__ void sb_f32_work(const SbSpmmArgs &a, int v)
     const int N = NRHS ? NRHS : a.n_rhs;
     const SbTask tk = sb_kload(a.tasks, v);
     if (tk.nrows == 0) return;               // filler of the task list
-    const SbMatBufs mb = sb_mat_bufs(a, tk.mat, a.scol);
+    const SbMatBufs mb = a.mats ? sb_kload(a.mats, tk.mat) : sb_mat_bufs(a, 0, a.scol);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if (tk.rounds > 0) {
         const int r0 = tk.r0 + tk.rows * wave;

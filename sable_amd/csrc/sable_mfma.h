@@ -38,14 +38,23 @@ typedef __attribute__((ext_vector_type(4))) float sb_f32x4;
 #define SB_SPLIT 3
 #endif
 
+// The 64-column workgroups of 256 threads (N above 64) run three to a compute
+// unit: registers for one k-step of A and X ahead and three waves per SIMD
+// (162 of 168) took the 50,000-row SpMM's dense blocks at N = 128 87.9 us,
+// two k-steps ahead at two waves per SIMD 91.3 us.
+#if SB_WG == 256 && SB_NRHS > 64 && SB_NRHS % 64 == 0
+#define SB_MFMA_THREE 1
+#else
+#define SB_MFMA_THREE 0
+#endif
 // k-steps of A loads in flight ahead of the MFMAs (A streams from HBM)
 #ifndef SB_MFMA_DEPTH
-#define SB_MFMA_DEPTH 2     // 1 to 4
+#define SB_MFMA_DEPTH (SB_MFMA_THREE ? 1 : 2)     // 1 to 4
 #endif
 // k-steps of X loads in flight ahead of their staging (X rows are shared by
 // many tiles and mostly come from L2): divides SB_MFMA_DEPTH
 #ifndef SB_MFMA_XDEPTH
-#define SB_MFMA_XDEPTH 2
+#define SB_MFMA_XDEPTH (SB_MFMA_THREE ? 1 : 2)
 #endif
 // the compiler's scheduling strategy for a k-step's basic block
 // (__builtin_amdgcn_iglp_opt), -1: none.  Strategy 3 ran the 50k SpMM at
@@ -81,9 +90,10 @@ typedef __attribute__((ext_vector_type(4))) float sb_f32x4;
 #define SB_MFMA_FENCE 0
 #endif
 // waves per SIMD the MFMA kernels are compiled for: two (256 registers per
-// lane, accumulators included), so two 256-thread workgroups share a CU
+// lane, accumulators included), so two 256-thread workgroups share a CU, or
+// three
 #ifndef SB_MFMA_WAVES
-#define SB_MFMA_WAVES 2
+#define SB_MFMA_WAVES (SB_MFMA_THREE ? 3 : 2)
 #endif
 
 __device__ __forceinline__ sb_bf16x8 sb_as_bf16x8(sb_u4 v) { return __builtin_bit_cast(sb_bf16x8, v); }
@@ -131,20 +141,20 @@ __device__ __forceinline__ void sb_split8(const float *f, sb_bf16x8 *t)
 // pointer with 32-bit offsets.
 typedef const __attribute__((address_space(1))) float *sb_gfloat;
 
-template <int WG, int UPT, int NRHS>
-__device__ __forceinline__ void sb_fetch_b(const float *X, int N, const int *xrow, int ncols, int ks,
+template <int WG, int UPT, int NC>
+__device__ __forceinline__ void sb_fetch_b(const float *X, int N, int nc, const int *xrow, int ncols, int ks,
                                            float (*f)[8])
 {
     (void)ncols;   // xrow holds row 0 for the columns past the piece (sb_expand_xrow_mfma)
     const sb_gfloat gX = (sb_gfloat)X;
-    constexpr bool EXACT = NRHS != 0 && UPT * WG == NRHS * 4;   // every unit in range
-    const int units = N * 4;
+    constexpr bool EXACT = NC != 0 && UPT * WG == NC * 4;   // every unit in range
+    const int units = nc * 4;
 #pragma unroll
     for (int uu = 0; uu < UPT; ++uu) {
         const int u = threadIdx.x + uu * WG;
         const int uc = EXACT || u < units ? u : 0;
-        const int kg = uc / N;
-        const int n = uc - kg * N;
+        const int kg = uc / nc;
+        const int n = uc - kg * nc;
         const int k0 = ks * 32 + kg * 8;
         const int4 ra = *reinterpret_cast<const int4 *>(xrow + k0);
         const int4 rb = *reinterpret_cast<const int4 *>(xrow + k0 + 4);
@@ -165,17 +175,17 @@ __device__ __forceinline__ void sb_expand_xrow_mfma(const SbXRange *__restrict__
     for (int i = threadIdx.x; i < pad; i += blockDim.x) xrow[ncols + i] = 0;
 }
 
-template <int WG, int UPT, int SPLIT, int NRHS, bool MASK = true>
-__device__ __forceinline__ void sb_store_b(int N, int ncols, int ks, float (*f)[8], uint16_t *B, int term_stride)
+template <int WG, int UPT, int SPLIT, int NC, bool MASK = true>
+__device__ __forceinline__ void sb_store_b(int nc, int ncols, int ks, float (*f)[8], uint16_t *B, int term_stride)
 {
-    constexpr bool EXACT = NRHS != 0 && UPT * WG == NRHS * 4;
-    const int units = N * 4;
+    constexpr bool EXACT = NC != 0 && UPT * WG == NC * 4;
+    const int units = nc * 4;
 #pragma unroll
     for (int uu = 0; uu < UPT; ++uu) {
         const int u = threadIdx.x + uu * WG;
         if (!EXACT && u >= units) continue;
-        const int kg = u / N;
-        const int n = u - kg * N;
+        const int kg = u / nc;
+        const int n = u - kg * nc;
         const int k0 = ks * 32 + kg * 8;
         float v[8];
 #pragma unroll
@@ -202,7 +212,7 @@ struct SbPasses {
 
 template <int WG, int NRHS, int SPLIT>
 struct SbMfmaCfg {
-    static constexpr int NMAX = NRHS ? NRHS : 256;
+    static constexpr int NMAX = NRHS ? SB_MFMA_COLS(NRHS, WG) : 256;        // columns of a workgroup
     static constexpr int NTMAX = NMAX / 16;
     static constexpr int NW = WG / 64;
     static constexpr int UNITS = SB_MFMA_UNITS1 ? 1 : SB_MFMA_UNITS(NMAX);   // row tiles per wavefront and pass
@@ -299,7 +309,7 @@ inline int sb_fixup_groups(const SbTile *fix, size_t nfix, int n_rhs)
 // its last one), so the compiler's waits stay exact.
 template <int WG, int NRHS, int SPLIT, int NU>
 __device__ __forceinline__ void sb_mfma_kloop(const SbSpmmArgs &a, const SbMatBufs &mb, const SbPiece &pc,
-                                              const int *umi, int N, int ntw, const int *xrow, uint16_t *B,
+                                              const int *umi, int N, int n0, int ntw, const int *xrow, uint16_t *B,
                                               sb_f32x4 (*acc)[SbMfmaCfg<WG, NRHS, SPLIT>::NTMAX])
 {
     using Cfg = SbMfmaCfg<WG, NRHS, SPLIT>;
@@ -311,7 +321,9 @@ __device__ __forceinline__ void sb_mfma_kloop(const SbSpmmArgs &a, const SbMatBu
     constexpr int NP = (Cfg::NTMAX + JB - 1) / JB;             // column pairs
     const int lane = threadIdx.x & 63;
     const int nb = lane & 15, kb = (lane >> 4) * 8;
-    const float *__restrict__ X = mb.x;
+    constexpr int NC = NRHS ? Cfg::NMAX : 0;
+    const int nc = NRHS ? Cfg::NMAX : N;                       // columns of this workgroup
+    const float *__restrict__ X = mb.x + n0;
     const int K = pc.ksteps;
     // a global-address-space pointer: loads through a generic pointer would
     // be FLAT loads, which count against the LDS counter as well, so every
@@ -356,12 +368,12 @@ __device__ __forceinline__ void sb_mfma_kloop(const SbSpmmArgs &a, const SbMatBu
     static_assert(SA <= DX, "the X slots cover the staged k-steps");
 #pragma unroll
     for (int j = 0; j < SA; ++j) {
-        sb_fetch_b<WG, Cfg::UPT, NRHS>(X, N, xrow, pc.ncols, j < K ? j : K - 1, xf[j % DX]);
-        sb_store_b<WG, Cfg::UPT, SPLIT, NRHS>(N, pc.ncols, j, xf[j % DX], B + j * Cfg::BUF_STRIDE, Cfg::TERM_STRIDE);
+        sb_fetch_b<WG, Cfg::UPT, NC>(X, N, nc, xrow, pc.ncols, j < K ? j : K - 1, xf[j % DX]);
+        sb_store_b<WG, Cfg::UPT, SPLIT, NC>(nc, pc.ncols, j, xf[j % DX], B + j * Cfg::BUF_STRIDE, Cfg::TERM_STRIDE);
     }
 #pragma unroll
     for (int j = SA; j < SA + DX; ++j)
-        sb_fetch_b<WG, Cfg::UPT, NRHS>(X, N, xrow, pc.ncols, j < K ? j : K - 1, xf[j % DX]);
+        sb_fetch_b<WG, Cfg::UPT, NC>(X, N, nc, xrow, pc.ncols, j < K ? j : K - 1, xf[j % DX]);
     split_a(ar[0]);
     load_a(ar[0], D < K ? D : K - 1);
     __syncthreads();
@@ -411,10 +423,10 @@ __device__ __forceinline__ void sb_mfma_kloop(const SbSpmmArgs &a, const SbMatBu
         // writes zeros nobody reads), then load the X values of k-step
         // ks + SA + DX into the slot it frees
         constexpr int xs = (sl + SA) % DX;
-        sb_store_b<WG, Cfg::UPT, SPLIT, NRHS, MASK>(N, pc.ncols, ks + SA, xf[xs],
+        sb_store_b<WG, Cfg::UPT, SPLIT, NC, MASK>(nc, pc.ncols, ks + SA, xf[xs],
                                                     B + ((ks + SA) & (Cfg::NBUF - 1)) * Cfg::BUF_STRIDE,
                                                     Cfg::TERM_STRIDE);
-        sb_fetch_b<WG, Cfg::UPT, NRHS>(X, N, xrow, pc.ncols, ks + SA + DX < K ? ks + SA + DX : K - 1, xf[xs]);
+        sb_fetch_b<WG, Cfg::UPT, NC>(X, N, nc, xrow, pc.ncols, ks + SA + DX < K ? ks + SA + DX : K - 1, xf[xs]);
 #if SB_MFMA_INTERLEAVE
         // issue order of the step: the first column pair's B reads, then
         // every MFMA followed by two VALU (the splits), a B read every
@@ -456,7 +468,7 @@ __device__ __forceinline__ void sb_mfma_kloop(const SbSpmmArgs &a, const SbMatBu
 // (unit, column tile) in that same lane order instead.
 template <int WG, int NRHS, int SPLIT, int NU>
 __device__ __forceinline__ void sb_mfma_pass(const SbSpmmArgs &a, const SbMatBufs &mb, const SbTile &tile,
-                                             const int *umi, int N, int nt, int mt, int *xrow, uint16_t *B)
+                                             const int *umi, int N, int n0, int nt, int mt, int *xrow, uint16_t *B)
 {
     using Cfg = SbMfmaCfg<WG, NRHS, SPLIT>;
     constexpr int NUA = NU > 0 ? NU : 1;
@@ -472,7 +484,7 @@ __device__ __forceinline__ void sb_mfma_pass(const SbSpmmArgs &a, const SbMatBuf
         __syncthreads();                               // previous piece done with xrow and B
         sb_expand_xrow_mfma(a.xr, pc.xr_begin, pc.xr_end, pc.ncols, xrow);
         __syncthreads();
-        sb_mfma_kloop<WG, NRHS, SPLIT, NU>(a, mb, pc, umi, N, nt, xrow, B, acc);
+        sb_mfma_kloop<WG, NRHS, SPLIT, NU>(a, mb, pc, umi, N, n0, nt, xrow, B, acc);
     }
     const bool split = tile.ksplit > 1;
 #pragma unroll
@@ -482,10 +494,10 @@ __device__ __forceinline__ void sb_mfma_pass(const SbSpmmArgs &a, const SbMatBuf
         for (int jj = 0; jj < Cfg::NTMAX; ++jj) {
             if (NRHS || jj < nt) {
                 if (split) {
-                    const int64_t blk = (int64_t)tile.part_blk + (int64_t)(tile.kpart * mt + umi[i]) * nt + jj;
+                    const int64_t blk = (int64_t)tile.part_blk + (int64_t)(tile.kpart * mt + umi[i]) * (N >> 4) + (n0 >> 4) + jj;
                     reinterpret_cast<SB_G sb_f32x4 *>(sb_gp(mb.part))[blk * 64 + lane] = acc[i][jj];
                 } else {
-                    const int col = jj * 16 + (lane & 15);
+                    const int col = n0 + jj * 16 + (lane & 15);
 #pragma unroll
                     for (int r = 0; r < 4; ++r)
                         if (rbase + r < tile.nrows)
@@ -506,13 +518,22 @@ __device__ __forceinline__ void sb_mfma_pass(const SbSpmmArgs &a, const SbMatBuf
 // the instance for the wavefront's unit count; every instance runs the same
 // barriers).
 template <int WG, int NRHS, int SPLIT>
-__device__ __forceinline__ void sb_spmm_mfma_tile(const SbSpmmArgs &a, int t, int *xrow, unsigned char *smem)
+__device__ __forceinline__ void sb_spmm_mfma_tile(const SbSpmmArgs &a, int v, int *xrow, unsigned char *smem)
 {
     using Cfg = SbMfmaCfg<WG, NRHS, SPLIT>;
     constexpr int NW = Cfg::NW;
     constexpr int UN = Cfg::UNITS;
     const int N = NRHS ? NRHS : a.n_rhs;
-    const int nt = N >> 4;
+    // item v: tile t, columns [n0, n0 + SB_MFMA_COLS).  The workgroups of a
+    // tile, which read the same A, are 8 apart: on one XCD, close in time
+    constexpr int NG = NRHS ? NRHS / Cfg::NMAX : 1;
+    int t = v, n0 = 0;
+    if constexpr (NG > 1) {
+        const int nt8 = a.ntiles / NG & ~7, k = v < nt8 * NG ? v >> 3 : v - nt8 * NG;
+        t = v < nt8 * NG ? (k / NG) * 8 + (v & 7) : nt8 + k / NG;
+        n0 = k % NG * Cfg::NMAX;
+    }
+    const int nt = NRHS ? Cfg::NTMAX : N >> 4;
     const SbTile tile = a.tiles[t];
     const int mt = (tile.nrows + 15) >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -537,11 +558,11 @@ __device__ __forceinline__ void sb_spmm_mfma_tile(const SbSpmmArgs &a, int t, in
             nact += act;
         }
         if (nact >= UN)
-            sb_mfma_pass<WG, NRHS, SPLIT, UN>(a, mb, tile, umi, N, nt, mt, xrow, B);
+            sb_mfma_pass<WG, NRHS, SPLIT, UN>(a, mb, tile, umi, N, n0, nt, mt, xrow, B);
         else if (UN > 1 && nact == 1)
-            sb_mfma_pass<WG, NRHS, SPLIT, 1>(a, mb, tile, umi, N, nt, mt, xrow, B);
+            sb_mfma_pass<WG, NRHS, SPLIT, 1>(a, mb, tile, umi, N, n0, nt, mt, xrow, B);
         else
-            sb_mfma_pass<WG, NRHS, SPLIT, 0>(a, mb, tile, umi, N, nt, mt, xrow, B);
+            sb_mfma_pass<WG, NRHS, SPLIT, 0>(a, mb, tile, umi, N, n0, nt, mt, xrow, B);
     }
 }
 
