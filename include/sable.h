@@ -223,6 +223,11 @@ int sable_mlp_backward(const float *params, int F, int H, int K, const float *X,
 /* dout = scale * 2 * (out - target) * mask, elementwise over n values */
 int sable_mlp_mse_grad(const float *out, const float *target, const float *mask, int64_t n,
                        float scale, float *dout);
+/* sable_mlp_forward, sable_mlp_mse_grad and sable_mlp_backward in one call
+ * (the same results; dout, out and hidden are written as by them) */
+int sable_mlp_gradient(const float *params, int F, int H, int K, const float *X, int n,
+                       const float *target, const float *mask, float scale, float *out,
+                       float *hidden, float *dout, float *grad);
 int sable_adam_step(float *params, const float *grad, float *m, float *v, int64_t n,
                     float lr, float beta1, float beta2, float eps, int step);
 

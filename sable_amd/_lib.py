@@ -106,6 +106,7 @@ _SIGS = {
     "sable_time_plans": (I32, [C.POINTER(P), I32, C.POINTER(P), C.POINTER(P), I32, I32, I64, F32P]),
     "sable_mlp_forward": (I32, [P, I32, I32, I32, P, I32, P, P]),
     "sable_mlp_backward": (I32, [P, I32, I32, I32, P, I32, P, P, P]),
+    "sable_mlp_gradient": (I32, [P, I32, I32, I32, P, I32, P, P, C.c_float, P, P, P, P]),
     "sable_mlp_mse_grad": (I32, [P, P, P, I64, C.c_float, P]),
     "sable_adam_step": (I32, [P, P, P, P, I64, C.c_float, C.c_float, C.c_float, C.c_float, I32]),
     "sable_bandwidth_probe": (I32, [I64, I32, F32P, F32P]),

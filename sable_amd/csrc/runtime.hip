@@ -1257,16 +1257,40 @@ int sable_group_destroy(SableGroup *g)
 
 // ---- router MLP
 
-int sable_mlp_forward(const float *params, int F, int H, int K, const float *X, int n, float *out,
-                      float *hidden)
+static int mlp_check(int F, int H, int K, int n)
 {
     if (g_device < 0) return fail(SABLE_ERR_NO_DEVICE, "sable_init not called");
     if (F <= 0 || H <= 0 || K <= 0 || n < 0 || H > 256 || F > 64 || K > 64)
         return fail(SABLE_ERR_INVALID, "MLP sizes out of range (F<=64, H<=256, K<=64)");
-    if (n == 0) return SABLE_OK;
-    hipLaunchKernelGGL(sb_mlp_forward_kernel, dim3((n + 255) / 256), dim3(256), 0, nullptr, params, F, H, K,
-                       X, n, out, hidden);
+    return SABLE_OK;
+}
+
+static int mlp_launch_forward(const float *params, int F, int H, int K, const float *X, int n, float *out, float *hidden,
+                              const float *target, const float *mask, float scale, float *dout)
+{
+    hipLaunchKernelGGL(sb_mlp_forward_kernel, dim3((n + SB_MLP_SPB - 1) / SB_MLP_SPB), dim3(256), 0, nullptr, params, F,
+                       H, K, X, n, out, hidden, target, mask, scale, dout);
     HIPOK(hipGetLastError());
+    return SABLE_OK;
+}
+
+static int mlp_launch_backward(const float *params, int F, int H, int K, const float *X, int n, const float *hidden,
+                               const float *dout, float *grad)
+{
+    // a workgroup per hidden unit and SB_MLP_BOUT of its gradients, one more for b2
+    const unsigned groups = (F + 1 + K + SB_MLP_BOUT - 1) / SB_MLP_BOUT;
+    hipLaunchKernelGGL(sb_mlp_backward_kernel, dim3(H + 1, groups), dim3(SB_MLP_BWG), 0, nullptr, params, F, H, K, X, n,
+                       hidden, dout, grad);
+    HIPOK(hipGetLastError());
+    return SABLE_OK;
+}
+
+int sable_mlp_forward(const float *params, int F, int H, int K, const float *X, int n, float *out,
+                      float *hidden)
+{
+    CHECKRC(mlp_check(F, H, K, n));
+    if (n == 0) return SABLE_OK;
+    CHECKRC(mlp_launch_forward(params, F, H, K, X, n, out, hidden, nullptr, nullptr, 0.f, nullptr));
     HIPOK(hipDeviceSynchronize());
     return SABLE_OK;
 }
@@ -1274,14 +1298,20 @@ int sable_mlp_forward(const float *params, int F, int H, int K, const float *X, 
 int sable_mlp_backward(const float *params, int F, int H, int K, const float *X, int n,
                        const float *hidden, const float *dout, float *grad)
 {
-    if (g_device < 0) return fail(SABLE_ERR_NO_DEVICE, "sable_init not called");
-    if (F <= 0 || H <= 0 || K <= 0 || n < 0 || H > 256 || F > 64 || K > 64)
-        return fail(SABLE_ERR_INVALID, "MLP sizes out of range (F<=64, H<=256, K<=64)");
-    const int64_t np = (int64_t)H * F + H + (int64_t)K * H + K;
-    // one workgroup per parameter chunk; deterministic fixed-order sums over samples
-    hipLaunchKernelGGL(sb_mlp_backward_kernel, dim3((unsigned)((np + 255) / 256)), dim3(256), 0, nullptr, params,
-                       F, H, K, X, n, hidden, dout, grad);
-    HIPOK(hipGetLastError());
+    CHECKRC(mlp_check(F, H, K, n));
+    CHECKRC(mlp_launch_backward(params, F, H, K, X, n, hidden, dout, grad));
+    HIPOK(hipDeviceSynchronize());
+    return SABLE_OK;
+}
+
+// forward, the masked MSE gradient and backward in two launches and one wait
+int sable_mlp_gradient(const float *params, int F, int H, int K, const float *X, int n, const float *target,
+                       const float *mask, float scale, float *out, float *hidden, float *dout, float *grad)
+{
+    CHECKRC(mlp_check(F, H, K, n));
+    if (!target || !mask || !dout) return fail(SABLE_ERR_INVALID, "null argument");
+    if (n > 0) CHECKRC(mlp_launch_forward(params, F, H, K, X, n, out, hidden, target, mask, scale, dout));
+    CHECKRC(mlp_launch_backward(params, F, H, K, X, n, hidden, dout, grad));
     HIPOK(hipDeviceSynchronize());
     return SABLE_OK;
 }

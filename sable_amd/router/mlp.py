@@ -75,11 +75,10 @@ class DeviceMLP:
 
     def gradient(self, Xd, Td, Md, n, scale):
         """Loss gradient w.r.t. the parameters into self.g (device)."""
-        out, hid = self.forward(Xd, n)
+        out, hid = self._buf("out", (n, self.K)), self._buf("hid", (n, self.H))
         dout = self._buf("dout", (n, self.K))
-        check(lib.sable_mlp_mse_grad(out.ptr, Td.ptr, Md.ptr, n * self.K, scale, dout.ptr))
-        check(lib.sable_mlp_backward(self.p.ptr, self.F, self.H, self.K, Xd.ptr, n, hid.ptr, dout.ptr,
-                                     self.g.ptr))
+        check(lib.sable_mlp_gradient(self.p.ptr, self.F, self.H, self.K, Xd.ptr, n, Td.ptr, Md.ptr, scale, out.ptr,
+                                     hid.ptr, dout.ptr, self.g.ptr))
         return out
 
     def adam(self, lr=3e-3, b1=0.9, b2=0.999, eps=1e-8):
