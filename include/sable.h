@@ -257,6 +257,15 @@ int sable_axis_cuts(const int64_t *indptr, const int32_t *indices, const double 
                     int64_t line_len, int kind, double threshold, uint8_t *cut, double *sim,
                     float *kernel_ms);
 
+/* Both axes of src/autopartition.py:34-68 cut_indices2 from one CSC matrix:
+ * col_cut (ncols + 1) as sable_axis_cuts gives it, row_cut (nrows + 1) as it
+ * gives it for the transpose, which is made on the device.  The rows of a
+ * column must be strictly ascending and below nrows, and neither axis may have
+ * more than 2^25 lines (SABLE_ERR_UNSUPPORTED otherwise).  kernel_ms (may be null): the time of the kernels. */
+int sable_partition_cuts(const int64_t *indptr, const int32_t *indices, const double *data, int64_t nrows,
+                         int64_t ncols, int kind, double threshold, uint8_t *col_cut, uint8_t *row_cut,
+                         float *kernel_ms);
+
 /* Block materialisation on the device (utils/convert_real_to_vbr.py:98-199,
  * convert_sparse_to_vbr: the reference slices every block on the host).
  * Input: a CSC matrix in host memory (indptr of ncols + 1, row indices below

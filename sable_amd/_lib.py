@@ -110,6 +110,7 @@ _SIGS = {
     "sable_mlp_mse_grad": (I32, [P, P, P, I64, C.c_float, P]),
     "sable_adam_step": (I32, [P, P, P, P, I64, C.c_float, C.c_float, C.c_float, C.c_float, I32]),
     "sable_bandwidth_probe": (I32, [I64, I32, F32P, F32P]),
+    "sable_partition_cuts": (I32, [P, P, P, I64, I64, I32, C.c_double, P, P, F32P]),
     "sable_axis_cuts": (I32, [P, P, P, I64, I64, I32, C.c_double, P, P, F32P]),
     "sable_inspect_create": (I32, [P, P, P, I64, I64, P, I32, P, I32, C.POINTER(P), C.POINTER(I64),
                                    C.POINTER(I64), F32P]),

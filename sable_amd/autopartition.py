@@ -170,10 +170,41 @@ def _axis_cuts_gpu(M, threshold, similarity, return_sim=False):
     return (cuts, sim[:max(n - 1, 0)]) if return_sim else cuts
 
 
+def _both_cuts_gpu(A, threshold, similarity):
+    """Both axes from one upload of the CSC matrix A, transposed on the GPU
+    (sable_partition_cuts), or None for a matrix this does not take: values
+    that are not real, columns whose rows are not strictly ascending
+    (duplicates are summed and rows sorted by the per-axis path), more than
+    2^25 lines, or more memory than is free.  The host transpose took a third
+    of a conversion's time."""
+    from . import runtime
+    from ._lib import lib, check, SableError, SABLE_ERR_OOM, SABLE_ERR_UNSUPPORTED
+    kind = _GPU_KIND.get(similarity)
+    if kind is None or A.dtype.kind not in "fiub" or min(A.shape) == 0 or max(A.shape) > 1 << 25:
+        return None
+    ip = np.ascontiguousarray(A.indptr, dtype=np.int64)
+    ix = np.ascontiguousarray(A.indices[:ip[-1]], dtype=np.int32)
+    v = np.ascontiguousarray(A.data[:ip[-1]], dtype=np.float64)
+    cuts = [np.zeros(n + 1, dtype=np.uint8) for n in (A.shape[1], A.shape[0])]
+    runtime.init()
+    try:
+        check(lib.sable_partition_cuts(ip.ctypes.data, ix.ctypes.data, v.ctypes.data, A.shape[0], A.shape[1], kind,
+                                       float(threshold), cuts[0].ctypes.data, cuts[1].ctypes.data, None))
+    except SableError as e:
+        if e.code not in (SABLE_ERR_UNSUPPORTED, SABLE_ERR_OOM):
+            raise
+        return None
+    return tuple(np.flatnonzero(c).tolist() for c in cuts)
+
+
 def cut_indices2(A, cut_threshold, similarity, device=False):
     """src/autopartition.py:34-68.  Returns (col_indices, row_indices).
     device=True computes both axes on the GPU (same result)."""
     A = scipy.sparse.csc_matrix(A)
+    if device:
+        both = _both_cuts_gpu(A, cut_threshold, similarity)
+        if both is not None:
+            return both
     axis = _axis_cuts_gpu if device else _axis_cuts
     cols = axis(A, cut_threshold, similarity)
     rows = axis(A.T.tocsc(), cut_threshold, similarity)

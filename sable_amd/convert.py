@@ -154,7 +154,7 @@ def _fetch_compressed(h, nb, nv2, nub, nnz, nrows, ncols, val_dtype):
                                            None))
     finally:
         lib.sable_compress_destroy(h)
-    val2 = val2.astype(val_dtype)
+    val2 = val2.astype(val_dtype, copy=False)
     if nnz < 0:
         return val2, indx2, ub, np.zeros(0, np.int64), np.zeros(0, np.int64), np.zeros(0, np.float64)
     # the index dtypes scipy gives the host construction (COO of int64 row /

@@ -1602,6 +1602,90 @@ int scan_exclusive(int64_t *d_in, int64_t n, int64_t *d_out, DevBufs &b)
 
 }  // namespace
 
+// Both axes of the partitioner from one upload: the columns as
+// sable_axis_cuts does them, the rows on the transpose made on the device.
+extern "C" int sable_partition_cuts(const int64_t *indptr, const int32_t *indices, const double *data, int64_t nrows,
+                                    int64_t ncols, int kind, double threshold, uint8_t *col_cut, uint8_t *row_cut,
+                                    float *kernel_ms)
+{
+    if (g_device < 0) return fail(SABLE_ERR_NO_DEVICE, "sable_init not called");
+    if (nrows <= 0 || ncols <= 0 || !indptr || !col_cut || !row_cut)
+        return fail(SABLE_ERR_INVALID, "bad partition_cuts arguments");
+    if (nrows > (1 << 25) || ncols > (1 << 25)) return fail(SABLE_ERR_UNSUPPORTED, "more than 2^25 lines");
+    if (kind < SB_SIM_S2 || kind > SB_SIM_S1) return fail(SABLE_ERR_INVALID, "unknown similarity kind");
+    if (indptr[0] != 0) return fail(SABLE_ERR_INVALID, "indptr[0] must be 0");
+    for (int64_t i = 0; i < ncols; ++i)
+        if (indptr[i + 1] < indptr[i]) return fail(SABLE_ERR_INVALID, "indptr must be nondecreasing");
+    const int64_t nnz = indptr[ncols];
+    if (nnz > 0 && (!indices || !data)) return fail(SABLE_ERR_INVALID, "null indices/data");
+    // as many column chunks as keep the counts within 64 MiB, at most 512
+    const int64_t most = std::min<int64_t>({512, ncols, std::max<int64_t>(1, (16 << 20) / nrows)});
+    const int64_t per = (ncols + most - 1) / most, nchunk = (ncols + per - 1) / per;
+    // one allocation, carved up (each allocation and release costs a wait)
+    int64_t at = 0;
+    auto carve = [&](int64_t bytes) {
+        const int64_t o = at;
+        at += (bytes + 255) & ~(int64_t)255;
+        return o;
+    };
+    const int64_t o_ip = carve((ncols + 1) * 8), o_ix = carve(nnz * 4), o_v = carve(nnz * 8), o_tip = carve((nrows + 1) * 8),
+                  o_tix = carve(nnz * 4), o_tv = carve(nnz * 8), o_cnt = carve(nchunk * nrows * 4),
+                  o_tot = carve((nrows + 1) * 8), o_cs = carve(ncols * 8), o_rs = carve(nrows * 8), o_cc = carve(ncols + 1),
+                  o_rc = carve(nrows + 1), o_bad = carve(4);
+    DevBufs b;
+    char *m = nullptr;
+    CHECKRC(b.alloc((void **)&m, at));
+    int64_t *ip = (int64_t *)(m + o_ip), *tip = (int64_t *)(m + o_tip), *tot = (int64_t *)(m + o_tot);
+    int32_t *ix = (int32_t *)(m + o_ix), *tix = (int32_t *)(m + o_tix), *cnt = (int32_t *)(m + o_cnt);
+    double *v = (double *)(m + o_v), *tv = (double *)(m + o_tv), *cs = (double *)(m + o_cs), *rs = (double *)(m + o_rs);
+    uint8_t *cc = (uint8_t *)(m + o_cc), *rc = (uint8_t *)(m + o_rc);
+    int *bad = (int *)(m + o_bad);
+    int h_bad = 0;
+    HIPOK(hipMemcpy(ip, indptr, (ncols + 1) * 8, hipMemcpyHostToDevice));
+    HIPOK(hipMemcpy(bad, &h_bad, 4, hipMemcpyHostToDevice));
+    if (nnz > 0) {
+        HIPOK(hipMemcpy(ix, indices, nnz * 4, hipMemcpyHostToDevice));
+        HIPOK(hipMemcpy(v, data, nnz * 8, hipMemcpyHostToDevice));
+    }
+    hipLaunchKernelGGL(sb_check_rows, dim3((unsigned)ncols), dim3(64), 0, nullptr, ip, ix, nrows, bad);
+    HIPOK(hipGetLastError());
+    HIPOK(hipMemcpy(&h_bad, bad, 4, hipMemcpyDeviceToHost));
+    if (h_bad) return fail(SABLE_ERR_UNSUPPORTED, "the rows of a column are not strictly ascending below nrows");
+    hipEvent_t e0, e1;
+    HIPOK(hipEventCreate(&e0));
+    HIPOK(hipEventCreate(&e1));
+    hipEventRecord(e0, nullptr);
+    auto axis = [&](const int64_t *p, const int32_t *x, const double *d, int64_t nlines, int64_t len, double *sim, uint8_t *cut) {
+        if (nlines > 1)
+            hipLaunchKernelGGL(sb_adjacent_sim, dim3((unsigned)((nlines - 1 + 3) / 4)), dim3(256), 0, nullptr, p, x, d,
+                               nlines, len, kind, sim);
+        hipLaunchKernelGGL(sb_cut_flags, dim3((unsigned)((nlines + 1 + 255) / 256)), dim3(256), 0, nullptr, p, sim, nlines,
+                           threshold, cut);
+    };
+    axis(ip, ix, v, ncols, nrows, cs, cc);
+    hipLaunchKernelGGL(sb_zero_i32, dim3(2048), dim3(256), 0, nullptr, cnt, nchunk * nrows);
+    hipLaunchKernelGGL(sb_count_rows, dim3((unsigned)nchunk), dim3(1024), 0, nullptr, ip, ix, nrows, ncols, per, cnt);
+    hipLaunchKernelGGL(sb_prefix_rows, dim3((unsigned)((nrows + 256) / 256)), dim3(256), 0, nullptr, cnt, nrows, nchunk, tot);
+    const int sc = scan_exclusive(tot, nrows + 1, tip, b);
+    hipLaunchKernelGGL(sb_place_rows, dim3((unsigned)nchunk), dim3(512), 0, nullptr, ip, ix, v, nrows, ncols, per, cnt, tip,
+                       tix, tv);
+    axis(tip, tix, tv, nrows, ncols, rs, rc);
+    hipEventRecord(e1, nullptr);
+    const hipError_t le = hipGetLastError();
+    const hipError_t se = hipEventSynchronize(e1);
+    float ms = 0.f;
+    hipEventElapsedTime(&ms, e0, e1);
+    hipEventDestroy(e0);
+    hipEventDestroy(e1);
+    CHECKRC(sc);
+    HIPOK(le);
+    HIPOK(se);
+    if (kernel_ms) *kernel_ms = ms;
+    HIPOK(hipMemcpy(col_cut, cc, ncols + 1, hipMemcpyDeviceToHost));
+    HIPOK(hipMemcpy(row_cut, rc, nrows + 1, hipMemcpyDeviceToHost));
+    return SABLE_OK;
+}
+
 int sable_inspect_create(const int64_t *indptr, const int32_t *indices, const double *data, int64_t nrows,
                          int64_t ncols, const int64_t *rpntr, int32_t nbr, const int64_t *cpntr, int32_t nbc,
                          SableInspect **out, int64_t *nblocks, int64_t *nval, float *device_ms)

@@ -198,3 +198,84 @@ __global__ void __launch_bounds__(256) sb_cut_flags(const int64_t *__restrict__ 
     }
     cut[p] = c;
 }
+
+// ---------------------------------------------------------------------------
+// Transpose of a CSC matrix for the row axis: stable (a row's entries in
+// column order), by counting.  The columns are cut into chunks, a workgroup
+// each: count the chunk's entries per row, prefix the counts over the chunks
+// (a row's entries of chunk c start there), then place the chunk's columns
+// one after another, the entries of a column (all of different rows) in
+// parallel.  HBM: 12 B per entry read twice and written once, the counts 4 B
+// per row and chunk four times; a workgroup's chain of columns is what takes
+// the time, so there are as many chunks as the counts' memory allows.
+// Measured on a 6,000-column matrix of 1.9 M entries: check 8, count 15,
+// prefix 46, place 64 us; both axes with the upload 1.2 ms, against 11.5 ms
+// with the transpose on the host and an upload per axis.
+
+// *bad becomes 1 if a column's rows are not strictly ascending in [0, nrows):
+// the transpose indexes by row.  A wavefront per column.
+__global__ void __launch_bounds__(64) sb_check_rows(const int64_t *__restrict__ ip, const int32_t *__restrict__ ix,
+                                                     int64_t nrows, int *__restrict__ bad)
+{
+    const int64_t e0 = ip[blockIdx.x], e1 = ip[blockIdx.x + 1];
+    for (int64_t e = e0 + threadIdx.x; e < e1; e += blockDim.x) {
+        const int64_t r = ix[e];
+        if (r < 0 || r >= nrows || (e > e0 && ix[e - 1] >= r)) *bad = 1;
+    }
+}
+
+__global__ void __launch_bounds__(256) sb_zero_i32(int32_t *__restrict__ p, int64_t n)
+{
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) p[i] = 0;
+}
+
+__global__ void __launch_bounds__(1024) sb_count_rows(const int64_t *__restrict__ ip, const int32_t *__restrict__ ix,
+                                                      int64_t nrows, int64_t ncols, int64_t per,
+                                                      int32_t *__restrict__ count)
+{
+    int32_t *c = count + (int64_t)blockIdx.x * nrows;
+    const int64_t j0 = (int64_t)blockIdx.x * per, j1 = j0 + per < ncols ? j0 + per : ncols;
+    for (int64_t e = ip[j0] + threadIdx.x; e < ip[j1]; e += blockDim.x) atomicAdd(&c[ix[e]], 1);
+}
+
+// count[c][r] becomes the entries of row r in the chunks before c; total[r]
+// all of them (total[nrows] = 0, for the scan)
+__global__ void __launch_bounds__(256) sb_prefix_rows(int32_t *__restrict__ count, int64_t nrows, int64_t nchunk,
+                                                      int64_t *__restrict__ total)
+{
+    const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (r > nrows) return;
+    int32_t s = 0;
+    if (r < nrows) {
+        for (int64_t c = 0; c < nchunk; c += 8) {       // eight loads in flight
+            int32_t v[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) v[k] = c + k < nchunk ? count[(c + k) * nrows + r] : 0;
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                if (c + k < nchunk) count[(c + k) * nrows + r] = s;
+                s += v[k];
+            }
+        }
+    }
+    total[r] = s;
+}
+
+__global__ void __launch_bounds__(512) sb_place_rows(const int64_t *__restrict__ ip, const int32_t *__restrict__ ix,
+                                                     const double *__restrict__ v, int64_t nrows, int64_t ncols,
+                                                     int64_t per, int32_t *count, const int64_t *__restrict__ tip,
+                                                     int32_t *__restrict__ tix, double *__restrict__ tv)
+{
+    int32_t *c = count + (int64_t)blockIdx.x * nrows;
+    const int64_t j0 = (int64_t)blockIdx.x * per, j1 = j0 + per < ncols ? j0 + per : ncols;
+    for (int64_t j = j0; j < j1; ++j) {
+        for (int64_t e = ip[j] + threadIdx.x; e < ip[j + 1]; e += blockDim.x) {
+            const int32_t r = ix[e];
+            const int32_t k = c[r];
+            c[r] = k + 1;
+            tix[tip[r] + k] = (int32_t)j;
+            tv[tip[r] + k] = v[e];
+        }
+        __syncthreads();                                // the next column may hold the same rows
+    }
+}
