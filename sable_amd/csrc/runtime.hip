@@ -1894,14 +1894,22 @@ int compress_on_device(const double *d_val, const int64_t *d_indx, const int64_t
     HIPOK(hipEventRecord(e0, nullptr));
     auto g256 = [](int64_t n) { return dim3((unsigned)((n + 255) / 256)); };
     HIPOK(hipMalloc((void **)&h->d_val2, std::max<int64_t>(h->nval2, 1) * sizeof(double)));
-    if (!dblk.empty())
-        hipLaunchKernelGGL(sb_gather_dense, dim3((unsigned)((dblk.size() + 3) / 4)), dim3(256), 0, nullptr, d_val,
-                           d_indx, d_dblk, d_indx2, (int64_t)dblk.size(), h->d_val2);
+    const int64_t ndense = (int64_t)dblk.size();
+    if (ndense > 0) {
+        const int parts =
+            (int)std::min<int64_t>(std::max<int64_t>(h->nval2 / ndense / SB_GATHER_VALUES, 1), SB_GATHER_PARTS);
+        hipLaunchKernelGGL(sb_gather_dense, dim3((unsigned)((ndense * parts + 3) / 4)), dim3(256), 0, nullptr, d_val,
+                           d_indx, d_dblk, d_indx2, ndense, parts, h->d_val2);
+    }
+    // values of sparse blocks per row: the columns a row's threads walk
+    const int64_t mean = (indx[nblocks] - h->nval2) / nrows;
+    const int segs = (int)std::min<int64_t>(std::max<int64_t>(mean / SB_CSR_COLS, 1), SB_CSR_SEGS);
+    const dim3 csr_grid((unsigned)((nrows + 63) / 64)), csr_block(64 * segs);
     int64_t nnz = 0;
     if (h->nub > 0) {
         hipLaunchKernelGGL(sb_part_map, g256(nrows), dim3(256), 0, nullptr, d_rp, nbr, nrows, d_rmap);
         HIPOK(hipMemsetAsync(d_last, 0, sizeof(int32_t), nullptr));
-        hipLaunchKernelGGL(sb_csr_rows, g256(nrows), dim3(256), 0, nullptr, d_val, d_indx, d_bindx, d_rp, d_cp,
+        hipLaunchKernelGGL(sb_csr_rows, csr_grid, csr_block, 0, nullptr, d_val, d_indx, d_bindx, d_rp, d_cp,
                            d_bb, d_be, d_sp, d_rmap, nrows, ncols, d_cnt, nullptr, nullptr, nullptr, d_last);
         HIPOK(hipMalloc((void **)&h->d_rowptr, (nrows + 1) * sizeof(int64_t)));
         CHECKRC(scan_exclusive(d_cnt, nrows, h->d_rowptr, b));
@@ -1918,7 +1926,7 @@ int compress_on_device(const double *d_val, const int64_t *d_indx, const int64_t
             h->nnz = nnz + (pad ? 1 : 0);
             HIPOK(hipMalloc((void **)&h->d_cols, h->nnz * sizeof(int64_t)));
             HIPOK(hipMalloc((void **)&h->d_vals, h->nnz * sizeof(double)));
-            hipLaunchKernelGGL(sb_csr_rows, g256(nrows), dim3(256), 0, nullptr, d_val, d_indx, d_bindx, d_rp, d_cp,
+            hipLaunchKernelGGL(sb_csr_rows, csr_grid, csr_block, 0, nullptr, d_val, d_indx, d_bindx, d_rp, d_cp,
                                d_bb, d_be, d_sp, d_rmap, nrows, ncols, d_cnt, h->d_rowptr, h->d_cols, h->d_vals,
                                d_last);
             if (pad) {

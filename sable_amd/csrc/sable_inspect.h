@@ -219,25 +219,34 @@ __global__ void __launch_bounds__(256) sb_scatter_values(const int32_t *__restri
 
 // ---- compressed (.vbrc) arrays on the device (reference:
 // utils/convert_real_to_vbr.py:18-96, convert_vbr_to_compressed, for given
-// routes).  Dense-routed blocks are gathered into val2 (one wavefront per
-// block); the nonzero values of sparse-routed blocks become a CSR matrix.
-// One thread per row walks its block row's sparse blocks in bindx order and,
-// inside a block, its columns in order, so every row comes out sorted by
-// column, as scipy's COO -> CSR conversion leaves it.  The reference's
-// padding entry (row nrows - 1, column ncols - 1, value 0, when the last row
-// or the last column holds no entry) is appended by the host.
+// routes).  Dense-routed blocks are gathered into val2, `parts` wavefronts per
+// block; the nonzero values of sparse-routed blocks become a CSR matrix.  Per
+// row, `segs` threads share the walk over its block row's sparse blocks in
+// bindx order and, inside a block, over its columns in order, a contiguous
+// part each, so every row comes out sorted by column, as scipy's COO -> CSR
+// conversion leaves it.  The reference's padding entry (row nrows - 1, column
+// ncols - 1, value 0, when the last row or the last column holds no entry) is
+// appended by the host.
+
+// Bound by the latency of a wavefront's chain of loads, so a block goes to
+// as many wavefronts as leave each about 512 values (SB_GATHER_PARTS at most;
+// one for small blocks, where a wavefront's launch is the cost): 160 us with
+// a wavefront per block, 17 us now, for the 210 dense blocks of a 6,007-row
+// matrix.
+#define SB_GATHER_PARTS 64
+#define SB_GATHER_VALUES 512
 
 __global__ void __launch_bounds__(256) sb_gather_dense(const double *__restrict__ val,
                                                        const int64_t *__restrict__ indx,
                                                        const int64_t *__restrict__ dblk,
-                                                       const int64_t *__restrict__ indx2, int64_t ndense,
+                                                       const int64_t *__restrict__ indx2, int64_t ndense, int parts,
                                                        double *__restrict__ val2)
 {
-    const int64_t d = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int64_t q = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6), d = q / parts;
     if (d >= ndense) return;
     const int64_t k = dblk[d], src = indx[k], n = indx[k + 1] - src, dst = indx2[d];
     // four loads in flight per lane, then their stores
-    for (int64_t e = threadIdx.x & 63; e < n; e += 256) {
+    for (int64_t e = (q - d * parts) * 256 + (threadIdx.x & 63); e < n; e += 256 * (int64_t)parts) {
         double x[4];
 #pragma unroll
         for (int u = 0; u < 4; ++u) x[u] = e + 64 * u < n ? val[src + e + 64 * u] : 0.0;
@@ -249,49 +258,77 @@ __global__ void __launch_bounds__(256) sb_gather_dense(const double *__restrict_
 
 // per row: the nonzero values of its sparse-routed blocks (count pass when
 // cols == nullptr, fill pass otherwise); lastcol is set when one of them is
-// in the last column
-__global__ void __launch_bounds__(256) sb_csr_rows(const double *__restrict__ val,
-                                                   const int64_t *__restrict__ indx,
-                                                   const int64_t *__restrict__ bindx,
-                                                   const int64_t *__restrict__ rpntr,
-                                                   const int64_t *__restrict__ cpntr,
-                                                   const int64_t *__restrict__ bpntrb,
-                                                   const int64_t *__restrict__ bpntre,
-                                                   const uint8_t *__restrict__ sparse, const int32_t *__restrict__ rmap,
-                                                   int64_t nrows, int64_t ncols, int64_t *__restrict__ cnt,
-                                                   const int64_t *__restrict__ rowptr, int64_t *__restrict__ cols,
-                                                   double *__restrict__ vals, int32_t *__restrict__ lastcol)
+// in the last column.  A workgroup holds 64 consecutive rows, so a
+// wavefront's loads of a column are contiguous, and blockDim.x / 64 segments
+// of their columns.  Bound by each thread's chain of column loads: one
+// segment per 32 sparse columns of the mean row, up to SB_CSR_SEGS.  On the
+// same matrix (248 sparse blocks) the count took 222 us with a thread per row
+// and takes 124, the fill 250 and 179; shares of 8 columns measured the same
+// there (125, 173).
+#define SB_CSR_SEGS 16
+#define SB_CSR_COLS 32
+
+__global__ void __launch_bounds__(64 * SB_CSR_SEGS)
+sb_csr_rows(const double *__restrict__ val, const int64_t *__restrict__ indx, const int64_t *__restrict__ bindx,
+            const int64_t *__restrict__ rpntr, const int64_t *__restrict__ cpntr, const int64_t *__restrict__ bpntrb,
+            const int64_t *__restrict__ bpntre, const uint8_t *__restrict__ sparse, const int32_t *__restrict__ rmap,
+            int64_t nrows, int64_t ncols, int64_t *__restrict__ cnt, const int64_t *__restrict__ rowptr,
+            int64_t *__restrict__ cols, double *__restrict__ vals, int32_t *__restrict__ lastcol)
 {
-    const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= nrows) return;
-    const int64_t a = rmap[r];
-    int64_t n = 0, pos = cols ? rowptr[r] : 0;
-    if (bpntrb[a] >= 0) {
-        const int64_t h = rpntr[a + 1] - rpntr[a], lr = r - rpntr[a];
-        for (int64_t k = bpntrb[a]; k < bpntre[a]; ++k) {
+    __shared__ int64_t part[SB_CSR_SEGS][64];
+    const int lane = (int)(threadIdx.x & 63), seg = (int)(threadIdx.x >> 6), segs = (int)(blockDim.x >> 6);
+    const int64_t r = (int64_t)blockIdx.x * 64 + lane;
+    const bool live = r < nrows;
+    const int64_t a = live ? rmap[r] : 0;
+    const int64_t kb = live && bpntrb[a] >= 0 ? bpntrb[a] : 0, ke = live && bpntrb[a] >= 0 ? bpntre[a] : 0;
+    const int64_t h = live ? rpntr[a + 1] - rpntr[a] : 0, lr = live ? r - rpntr[a] : 0;
+    // columns of the row's sparse blocks, and this segment's part of them
+    int64_t total = 0;
+    for (int64_t k = kb; k < ke; ++k)
+        if (sparse[k]) total += cpntr[bindx[k] + 1] - cpntr[bindx[k]];
+    const int64_t s0 = total * seg / segs, s1 = total * (seg + 1) / segs;
+    // calls f(column, value) for the segment's nonzero values in order
+    auto walk = [&](auto f) {
+        int64_t at = 0;
+        for (int64_t k = kb; k < ke && at < s1; ++k) {
             if (!sparse[k]) continue;
             const int64_t b = bindx[k], c0 = cpntr[b], w = cpntr[b + 1] - c0;
+            const int64_t from = s0 > at ? s0 - at : 0, to = s1 - at < w ? s1 - at : w;
+            at += w;
             const double *__restrict__ blk = val + indx[k] + lr;
             // eight columns per step, their loads issued together (a
-            // column past the block reads its last column again)
-            for (int64_t c = 0; c < w; c += 8) {
+            // column past the part reads its last column again)
+            for (int64_t c = from; c < to; c += 8) {
                 double xv[8];
 #pragma unroll
-                for (int u = 0; u < 8; ++u) xv[u] = blk[(c + u < w ? c + u : w - 1) * h];
+                for (int u = 0; u < 8; ++u) xv[u] = blk[(c + u < to ? c + u : to - 1) * h];
 #pragma unroll
-                for (int u = 0; u < 8; ++u) {
-                    if (c + u >= w || xv[u] == 0.0) continue;
-                    if (cols) {
-                        cols[pos] = c0 + c + u;
-                        vals[pos] = xv[u];
-                        ++pos;
-                    } else {
-                        ++n;
-                        if (c0 + c + u == ncols - 1) *lastcol = 1;
-                    }
-                }
+                for (int u = 0; u < 8; ++u)
+                    if (c + u < to && xv[u] != 0.0) f(c0 + c + u, xv[u]);
             }
         }
+    };
+    int64_t n = 0;
+    walk([&](int64_t c, double) {
+        ++n;
+        if (!cols && c == ncols - 1) *lastcol = 1;
+    });
+    part[seg][lane] = n;
+    __syncthreads();
+    if (!live) return;
+    if (!cols) {
+        if (seg == 0) {
+            int64_t s = 0;
+            for (int q = 0; q < segs; ++q) s += part[q][lane];
+            cnt[r] = s;
+        }
+        return;
     }
-    if (!cols) cnt[r] = n;
+    int64_t pos = rowptr[r];
+    for (int q = 0; q < seg; ++q) pos += part[q][lane];
+    walk([&](int64_t c, double x) {
+        cols[pos] = c;
+        vals[pos] = x;
+        ++pos;
+    });
 }
