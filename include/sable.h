@@ -88,8 +88,10 @@ typedef struct {
                                  (FP32-level, default); 2 = hi+lo, 3 passes */
     int32_t min_tiles;        /* tiles wanted at least: while a plan has fewer, its
                                  tile_bytes is halved (down to 16 KiB) so small
-                                 matrices still fill the device; 0 = 1024 for
-                                 SpMV, 256 for SpMM */
+                                 matrices still fill the device; 0 = 256 for
+                                 SpMM, and for SpMV a tile target (at most
+                                 tile_bytes) that follows the matrix and the
+                                 workgroups the device holds at once */
     int32_t mfma_kchunk;      /* SpMM MFMA tiles: at most about this many 32-column
                                  k-steps per work item; a longer row tile is split
                                  along k into chunks whose partial sums a fixup
@@ -125,7 +127,8 @@ typedef struct {
     int64_t fixup_bytes;      /* partial sums written and read back per launch */
     int64_t nspans;           /* SpMV row spans: tiles of several short block rows,
                                  every block on the sparse path (0 when they would
-                                 leave the plan below min_tiles) */
+                                 leave the plan below min_tiles, or by
+                                 default below a tile per CU) */
 } SablePlanStats;
 
 /* Library. */

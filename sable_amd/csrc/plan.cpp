@@ -44,7 +44,8 @@ SablePlanOpts normalize_opts(const SablePlanOpts *in)
     if (o.mfma_split != 2) o.mfma_split = 3;
     // SpMV tiles are light (stream-bound); SpMM tiles carry MFMA work and
     // gain from tall tiles (each staged X k-step serves every row)
-    if (o.min_tiles <= 0) o.min_tiles = (o.op == SABLE_OP_SPMV) ? 1024 : 256;
+    // (0 for SpMV: the tile target follows the matrix, see build_host_plan)
+    if (o.min_tiles <= 0) o.min_tiles = (o.op == SABLE_OP_SPMV) ? 0 : 256;
     // k-split of MFMA row tiles only on request: on the 50k SpMM at N = 128
     // 32-k-step chunks measured 1-3.5 % slower than unsplit tiles (the fixup
     // launch and the partial-sum traffic outweigh the shorter chains)
@@ -374,26 +375,100 @@ double emit_wave_slices(HostPlan &P, SablePlanStats &S, SbTile &t, const std::ve
 namespace {
 int build_host_plan_once(const SableVbr &v, const uint8_t *route, const SablePlanOpts &o, bool spans, HostPlan &P,
                          std::string &err);
+
+// min_tiles asked for: the tile target is halved until there are that many
+// tiles (or tiles are 16 KiB).
+int build_with_min_tiles(const SableVbr &v, const uint8_t *route, const SablePlanOpts &o, bool spans, HostPlan &P,
+                         std::string &err)
+{
+    SablePlanOpts oo = o;
+    for (;;) {
+        const int rc = build_host_plan_once(v, route, oo, spans, P, err);
+        if (rc) return rc;
+        if ((int64_t)P.tiles.size() >= oo.min_tiles || oo.tile_bytes <= 16 * 1024) return SABLE_OK;
+        oo.tile_bytes = std::max<int64_t>(16 * 1024, oo.tile_bytes / 2);
+    }
+}
+
+// SpMV on its own: tile_bytes bounds the tile target, which is set by the
+// workgroups the device holds at once (768 of 512 threads).  A tile costs
+// several dependent round trips however small it is, so one round of tiles
+// that all fit is best where the block rows allow it; a second, nearly empty
+// round costs as much as the first.  The target is 1.4 times the bytes per
+// slot; if that gives more tiles than slots, up to 2.2 times, where the tiles
+// then fit.  Beyond that the largest tiles are longer than a second round.
+// Measured with cold caches, 512 threads, in us, against a target halved until
+// 1024 tiles:
+//   20,011 rows, 12 MB: 12.0 -> 10.4 (783 tiles -> 454)
+//   30,011 rows, 25 MB: 17.1 -> 12.9 (1066 -> 766)
+//   40,000 rows, 41 MB: 21.0 -> 14.6 (1382 -> 766)
+//   70,000 rows, 70 MB: 23.1 -> 20.5 (1383 -> 745)
+//   80,000 rows, 107 MB: 29.1 -> 28.0 (1180 -> 960; 758 tiles: 31.4)
+//   100,000 rows, 276 MB: 54.5 -> 53.2 (1089 -> 1111)
+// A tile of fewer than 32 KiB is shorter than its fixed cost (6,000 rows,
+// 6 MB: 9.6 us with 349 tiles of 16 KiB, 8.5 with 198 of 32 KiB) unless it is
+// one of few (1,000 rows: 6.8 us with 40 tiles, 7.1 with 26).
+int build_for_slots(const SableVbr &v, const uint8_t *route, const SablePlanOpts &o, bool spans, HostPlan &P,
+                    std::string &err)
+{
+    int rc = validate_vbr(v, err);
+    if (rc) return rc;
+    const int64_t slots = std::max<int64_t>(1, (int64_t)SB_SIMDS * std::max(2, SB_SPMV_WAVES(o.unroll)) * 64 / o.wg);
+    // value bytes of the plan: 4 per dense value, 6 per sparse entry
+    int64_t bytes = 0;
+    for (int64_t k = 0; k < v.nblocks; ++k) {
+        const float *b = v.val + v.indx[k];
+        const int64_t n = v.indx[k + 1] - v.indx[k];
+        if (route && route[k] == SABLE_ROUTE_SPARSE) {
+            int64_t c = 0;
+            for (int64_t e = 0; e < n; ++e) c += b[e] != 0.f;
+            bytes += 6 * c;
+        } else {
+            bytes += 4 * n;
+        }
+    }
+    const double share = (double)bytes / (double)slots;
+    SablePlanOpts oo = o;
+    auto target = [&](double bytes) {
+        oo.tile_bytes = std::min<int64_t>(o.tile_bytes, std::max<int64_t>((int64_t)bytes, 32 * 1024));
+        return oo.tile_bytes;
+    };
+    target(1.4 * share);
+    rc = build_host_plan_once(v, route, oo, spans, P, err);
+    if (rc) return rc;
+    if ((int64_t)P.tiles.size() * 2 < SB_CUS && oo.tile_bytes == 32 * 1024) {
+        oo.tile_bytes = 16 * 1024;
+        return build_host_plan_once(v, route, oo, spans, P, err);
+    }
+    for (const double f : {1.6, 1.9, 2.2}) {
+        if ((int64_t)P.tiles.size() <= slots || f * share > (double)o.tile_bytes) return SABLE_OK;
+        if (f * share <= 32.0 * 1024) continue;
+        target(f * share);
+        HostPlan Q;
+        rc = build_host_plan_once(v, route, oo, spans, Q, err);
+        if (rc) return rc;
+        if ((int64_t)Q.tiles.size() <= slots) {
+            P = std::move(Q);
+            return SABLE_OK;
+        }
+    }
+    return SABLE_OK;
+}
 }
 
 int build_host_plan(const SableVbr &v, const uint8_t *route, const SablePlanOpts &o,
                     HostPlan &P, std::string &err)
 {
-    // Small matrices: halve the tile target until there are min_tiles tiles
-    // (or tiles are 16 KiB), so the launch still spreads over the device.
     // Row spans trade tiles for less fixed cost per row; a plan they would
-    // leave below min_tiles is built without them (a small matrix launched
+    // leave with too few tiles is built without them (a small matrix launched
     // on its own needs the parallelism; plans built for a group take
     // min_tiles 1 and keep them).
     for (int spans = 1; spans >= 0; --spans) {
-        SablePlanOpts oo = o;
-        for (;;) {
-            const int rc = build_host_plan_once(v, route, oo, spans != 0, P, err);
-            if (rc) return rc;
-            if ((int64_t)P.tiles.size() >= oo.min_tiles || oo.tile_bytes <= 16 * 1024) break;
-            oo.tile_bytes = std::max<int64_t>(16 * 1024, oo.tile_bytes / 2);
-        }
-        if ((int64_t)P.tiles.size() >= o.min_tiles || !P.stats.nspans) return SABLE_OK;
+        const int rc = o.min_tiles > 0 ? build_with_min_tiles(v, route, o, spans != 0, P, err)
+                                       : build_for_slots(v, route, o, spans != 0, P, err);
+        if (rc) return rc;
+        const int64_t few = o.min_tiles > 0 ? o.min_tiles : SB_CUS;
+        if ((int64_t)P.tiles.size() >= few || !P.stats.nspans) return SABLE_OK;
     }
     return SABLE_OK;
 }

@@ -54,6 +54,14 @@ struct SbTile {
 #define SB_SPUNROLL 2
 #define SB_SPMV_INFLIGHT 1
 
+// The waves per SIMD the SpMV kernel is compiled for (its VGPR budget) given
+// the dense unroll: 80 VGPRs (6 waves) at unroll 2, 96 (5 waves) at unroll 4.
+// SB_SPMV_MINWAVES > 0 sets it for every unroll.
+#ifndef SB_SPMV_MINWAVES
+#define SB_SPMV_MINWAVES 0
+#endif
+#define SB_SPMV_WAVES(U) (SB_SPMV_MINWAVES > 0 ? SB_SPMV_MINWAVES : (U) <= 2 ? 6 : (U) <= 4 ? 5 : 1)
+
 // SpMV row spans: runs of short block rows (at most SB_SPMV_SHORT_ROWS rows
 // and SB_SPMV_SHORT_VALUES stored values each) are planned as one tile of at
 // most SB_SPMV_SPAN_ROWS rows (and the workgroup size) and
@@ -66,6 +74,7 @@ struct SbTile {
 // the device hands workgroups to its XCDs round robin
 #define SB_XCDS 8
 #define SB_SIMDS 1024
+#define SB_CUS 256
 
 // FP32 SpMM.  A tile with dense pieces is cut into workgroups of 64 columns
 // of Y, each wavefront taking 32 (or 16) of its rows; a tile without, into workgroups

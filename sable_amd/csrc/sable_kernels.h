@@ -220,14 +220,6 @@ __device__ __forceinline__ void sb_for_tiles(int ntiles, int mode, int32_t *queu
 // Row r's result is (dense partial sums of the M column groups, in group
 // order) + (sparse sums, piece by piece): deterministic, no atomics.
 
-// The waves per SIMD the SpMV kernel is compiled for (its VGPR budget) given
-// the dense unroll: 80 VGPRs (6 waves) at unroll 2, 96 (5 waves) at unroll 4.
-// SB_SPMV_MINWAVES > 0 sets it for every unroll.
-#ifndef SB_SPMV_MINWAVES
-#define SB_SPMV_MINWAVES 0
-#endif
-#define SB_SPMV_WAVES(U) (SB_SPMV_MINWAVES > 0 ? SB_SPMV_MINWAVES : (U) <= 2 ? 6 : (U) <= 4 ? 5 : 1)
-
 struct SbStreamLane {
     int c0, c1, c2, c3;    // column offsets of this lane's four elements
 };
