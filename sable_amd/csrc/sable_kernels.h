@@ -255,14 +255,14 @@ __device__ __forceinline__ void sb_dense_fma(const sb_f4 *v, const float *xs, co
     }
 }
 
-// Streams one dense piece whose x slice starts at xs.
+// Streams one dense piece whose x slice starts at xs; cur holds its first
+// batch.
 template <int UNROLL>
 __device__ __forceinline__ void sb_dense_piece(const SB_G sb_f4 *__restrict__ P, int nq, int tpar, int M, int ncols,
-                                               const float *xs, const SbStreamLane &L, float &a0, float &a1,
-                                               float &a2, float &a3)
+                                               const float *xs, const SbStreamLane &L, sb_f4 *cur, float &a0,
+                                               float &a1, float &a2, float &a3)
 {
     const int tid = threadIdx.x;
-    if (tid >= tpar || tid >= nq) return;
     const int nmine = (nq - 1 - tid) / tpar + 1;             // float4 loads of this lane
     const int nbatch = (nmine + UNROLL - 1) / UNROLL;
     // The register copy cur = nxt waits for the batch it copies, so one
@@ -271,8 +271,7 @@ __device__ __forceinline__ void sb_dense_piece(const SB_G sb_f4 *__restrict__ P,
     // per SIMD, two 512-thread workgroups per CU) and measured no faster on
     // the 100k matrix: the kernel runs at about 85 % of a cold streaming
     // read of the same bytes either way.
-    sb_f4 cur[UNROLL], nxt[UNROLL];
-    sb_dense_load<UNROLL>(P, nq, tid, tpar, cur);
+    sb_f4 nxt[UNROLL];
     for (int b = 0; b < nbatch; ++b) {
         // always prefetch (the batch after the last one reads the zero float4)
         sb_dense_load<UNROLL>(P, nq, tid + (b + 1) * UNROLL * tpar, tpar, nxt);
@@ -284,10 +283,11 @@ __device__ __forceinline__ void sb_dense_piece(const SB_G sb_f4 *__restrict__ P,
 
 // Stages a group's x slices into xs through its slot map (x column per slot,
 // -1 for the zero pads): two dependent loads per slot, 4 slots in flight per
-// thread, no search over descriptors.
-template <int WG>
+// thread, no search over descriptors.  issue() runs while the first map
+// loads are under way.
+template <int WG, typename Issue>
 __device__ __forceinline__ void sb_stage_map(const SB_G int32_t *__restrict__ map, int total,
-                                             const SB_G float *__restrict__ x, float *xs)
+                                             const SB_G float *__restrict__ x, float *xs, Issue issue)
 {
     for (int i0 = 0; i0 < total; i0 += 4 * WG) {
         int m[4];
@@ -296,6 +296,7 @@ __device__ __forceinline__ void sb_stage_map(const SB_G int32_t *__restrict__ ma
             const int i = i0 + u * WG + (int)threadIdx.x;
             m[u] = i < total ? __builtin_nontemporal_load(&map[i]) : -1;
         }
+        if (i0 == 0) issue();
         float v[4];
 #pragma unroll
         for (int u = 0; u < 4; ++u) v[u] = m[u] >= 0 ? x[m[u]] : 0.f;
@@ -323,6 +324,9 @@ __device__ __forceinline__ void sb_sparse_slice(const SB_G float *__restrict__ s
     const int off = tab[2 * slice];
     const int nst = tab[2 * slice + 1];
     if (nst <= 0) return;
+    const int i = slice * (64 >> glog) + (lane >> glog);
+    const bool owner = (lane & ((1 << glog) - 1)) == 0 && i < hs;
+    const int row = owner ? map[i] : 0;
     const SB_G sb_f4 *__restrict__ V = reinterpret_cast<const SB_G sb_f4 *>(sval) + (int64_t)off * 64 + lane;
     const SB_G sb_u2 *__restrict__ I = reinterpret_cast<const SB_G sb_u2 *>(sidx) + (int64_t)off * 64 + lane;
     const unsigned padpair = (unsigned)pad | ((unsigned)pad << 16);
@@ -361,30 +365,22 @@ __device__ __forceinline__ void sb_sparse_slice(const SB_G float *__restrict__ s
         }
     }
     for (int m = 1; m < (1 << glog); m <<= 1) acc += __shfl_xor(acc, m, 64);
-    const int i = slice * (64 >> glog) + (lane >> glog);
-    if ((lane & ((1 << glog) - 1)) == 0 && i < hs) spy[map[i]] += acc;
+    if (owner) spy[row] += acc;
 }
 
 template <int WG, int UNROLL, int XCAP>
 __device__ __forceinline__ void sb_spmv_tile(const SbSpmvArgs &a, int t, float *xs, float *red, float *spy)
 {
     const int tid = threadIdx.x;
-    const SbTile tile = a.tiles[t];
+    const SbTile tile = sb_kload(a.tiles, __builtin_amdgcn_readfirstlane(t));
     const int hs = tile.nrows;
     const int tpar = tile.dense_tpar;
     const int M = tile.dense_mcols;
-    const SbMatBufs mb = sb_mat_bufs(a, tile.mat, a.xmap);
+    const SbMatBufs mb = a.mats ? sb_kload(a.mats, tile.mat) : sb_mat_bufs(a, 0, a.xmap);
     const SB_G float *__restrict__ x = sb_gp(mb.x);
     SB_G float *__restrict__ y = sb_gp(mb.y);
 
     SbStreamLane L;
-    {
-        const int p0 = 4 * tid;
-        L.c0 = p0 / hs;
-        L.c1 = (p0 + 1) / hs;
-        L.c2 = (p0 + 2) / hs;
-        L.c3 = (p0 + 3) / hs;
-    }
     float a0 = 0.f, a1 = 0.f, a2 = 0.f, a3 = 0.f;
     if (tid < hs) spy[tid] = 0.f;   // before the first staging barrier; sparse row owners add after it
     // roles: lanes tid < tpar stream the dense pieces; the last nsw
@@ -400,22 +396,53 @@ __device__ __forceinline__ void sb_spmv_tile(const SbSpmvArgs &a, int t, float *
         // staging group [pb, pe), formed by the host (stage_len <= XCAP + 4
         // slots); the first group's map offset and length come with the
         // tile, so its map loads need not wait for the piece descriptor
-        const SbPiece first = a.pieces[pb];
+        const SbPiece first = sb_kload(a.pieces, pb);
+        const SbPiece second = sb_kload(a.pieces, pb + 1);    // the array has slack behind it
         const int smap = head ? tile.stage_map : first.xmap_off;
         const int slen = head ? tile.stage_len : first.stage_len;
-        head = false;
         if (slen > XCAP + 4) break;            // never built (the host and kernel choice check)
         __syncthreads();                       // previous group done with xs
-        sb_stage_map<WG>(sb_gp(mb.xmap) + smap, slen, x, xs);
+        // A tile is a chain of round trips (tile, pieces, map, x, values), so
+        // what needs no x goes ahead of it: the first batch of the group's
+        // first dense piece (its first or second piece, else it is loaded
+        // when its turn comes) is in flight while x is staged.  With the
+        // descriptors in scalar registers (nothing spilled; 8 VGPRs were)
+        // this took the kernel from 5.0 to 4.0 us at 1,000 rows, 9.8 to 7.6
+        // at 30,011 and 49.8 to 47.8 at 100,000 (warm caches).
+        const int ahead = first.kind == SB_PIECE_DENSE                                       ? pb
+                          : second.kind == SB_PIECE_DENSE && first.grp_end > pb + 1 ? pb + 1
+                                                                                             : -1;
+        // (Without one, and on the lanes past tpar, the loads read some 16
+        // bytes that exist: a branch here would make x wait for the batch.)
+        const int64_t aoff = ahead == pb ? first.data_off : second.data_off;
+        const int anq = ahead < 0 ? 0 : (hs * (ahead == pb ? first.ncols : second.ncols) + 3) >> 2;
+        const SB_G sb_f4 *AP = ahead < 0 ? reinterpret_cast<const SB_G sb_f4 *>(sb_gp(a.tiles))
+                                         : reinterpret_cast<const SB_G sb_f4 *>(sb_gp(mb.dval) + aoff);
+        sb_f4 cur[UNROLL];
+        sb_stage_map<WG>(sb_gp(mb.xmap) + smap, slen, x, xs, [&] {
+            sb_dense_load<UNROLL>(AP, anq, tid < tpar ? tid : anq, tpar, cur);
+            if (head) {
+                const int p0 = 4 * tid;
+                L.c0 = p0 / hs;
+                L.c1 = (p0 + 1) / hs;
+                L.c2 = (p0 + 2) / hs;
+                L.c3 = (p0 + 3) / hs;
+            }
+        });
+        head = false;
         __syncthreads();
         const int pe = first.grp_end;
         if (pe <= pb) break;                   // never built
         int base = 0;
         for (int p = pb; p < pe; ++p) {
-            const SbPiece pc = a.pieces[p];
+            const SbPiece pc = sb_kload(a.pieces, p);
             if (pc.kind == SB_PIECE_DENSE) {
-                sb_dense_piece<UNROLL>(reinterpret_cast<const SB_G sb_f4 *>(sb_gp(mb.dval) + pc.data_off),
-                                       (hs * pc.ncols + 3) >> 2, tpar, M, pc.ncols, xs + base, L, a0, a1, a2, a3);
+                const SB_G sb_f4 *P = reinterpret_cast<const SB_G sb_f4 *>(sb_gp(mb.dval) + pc.data_off);
+                const int nq = (hs * pc.ncols + 3) >> 2;
+                if (tid < tpar && tid < nq) {
+                    if (p != ahead) sb_dense_load<UNROLL>(P, nq, tid, tpar, cur);
+                    sb_dense_piece<UNROLL>(P, nq, tpar, M, pc.ncols, xs + base, L, cur, a0, a1, a2, a3);
+                }
             } else if (sw >= 0) {
                 // this wavefront's slices sw, sw + nsw, ...
                 for (int sl = sw; sl < nsl; sl += nsw) {
