@@ -160,7 +160,13 @@ class Plan:
         given = {"wg": wg, "tile_bytes": tile_bytes, "mode": mode, "unroll": unroll}
         if tuned:
             from .autotune import tuned_options
-            for k, v in tuned_options(op, n_rhs).items():
+            best = tuned_options(op, n_rhs)
+            if op == "spmv" and wg is not None and wg != best.get("wg"):
+                # measured for another workgroup size: 512 KiB tiles, right
+                # for 512 threads, are 64 round trips of 256 (the library's
+                # default follows the threads)
+                best.pop("tile_bytes", None)
+            for k, v in best.items():
                 if k in given and given[k] is None:
                     given[k] = v
         wg = given["wg"] or 256
