@@ -970,10 +970,17 @@ __device__ __forceinline__ void sb_spmm_f32_body(const SbSpmmArgs &a)
 __device__ __forceinline__ void sb_expand_xrow(const SbXRange *__restrict__ xr, int r0, int r1, int *xrow)
 {
     int base = 0;
-    for (int r = r0; r < r1; ++r) {
-        const SB_G SbXRange *g = sb_gp(xr) + r;
-        const int col0 = g->col0, len = g->len;
-        for (int i = threadIdx.x; i < len; i += blockDim.x) xrow[base + i] = col0 + i;
-        base += len;
+    for (int r = r0; r < r1; r += 4) {
+        // four ranges per round trip (the array has slack behind it)
+        struct alignas(8) Four {
+            SbXRange q[4];
+        };
+        const Four f = sb_kload(reinterpret_cast<const Four *>(xr + r), 0);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int len = r + k < r1 ? f.q[k].len : 0;
+            for (int i = threadIdx.x; i < len; i += blockDim.x) xrow[base + i] = f.q[k].col0 + i;
+            base += len;
+        }
     }
 }

@@ -309,7 +309,7 @@ inline int sb_fixup_groups(const SbTile *fix, size_t nfix, int n_rhs)
 // its last one), so the compiler's waits stay exact.
 template <int WG, int NRHS, int SPLIT, int NU>
 __device__ __forceinline__ void sb_mfma_kloop(const SbSpmmArgs &a, const SbMatBufs &mb, const SbPiece &pc,
-                                              const int *umi, int N, int n0, int ntw, const int *xrow, uint16_t *B,
+                                              const int *umi, int N, int n0, int ntw, int *xrow, uint16_t *B,
                                               sb_f32x4 (*acc)[SbMfmaCfg<WG, NRHS, SPLIT>::NTMAX])
 {
     using Cfg = SbMfmaCfg<WG, NRHS, SPLIT>;
@@ -359,8 +359,15 @@ __device__ __forceinline__ void sb_mfma_kloop(const SbSpmmArgs &a, const SbMatBu
                 bt[c][s] = *reinterpret_cast<const sb_bf16x8 *>(Bc + s * Cfg::TERM_STRIDE + n * SB_KP + kb);
         }
     };
+    // A needs no X row, so its first loads are in flight while they are laid
+    // out (and the ranges come four per scalar load): the batch of 16 members
+    // at N = 16 39.9 -> 36.6 us, the 50,000-row SpMM's MFMA launch at N = 128
+    // 88 -> 86 us
 #pragma unroll
     for (int sl = 0; sl < D; ++sl) load_a(ar[sl], sl < K ? sl : K - 1);
+    __syncthreads();                                   // previous piece done with xrow and B
+    sb_expand_xrow_mfma(a.xr, pc.xr_begin, pc.xr_end, pc.ncols, xrow);
+    __syncthreads();
     // staged k-steps ahead of the one multiplied: 1 with two buffers, 2 with
     // four (k-step s in buffer s % NBUF; the barrier after every
     // (NBUF / 2)-th step orders each buffer's writes after its last reads)
@@ -479,11 +486,9 @@ __device__ __forceinline__ void sb_mfma_pass(const SbSpmmArgs &a, const SbMatBuf
 #pragma unroll
         for (int j = 0; j < Cfg::NTMAX; ++j) acc[u][j] = sb_f32x4{0.f, 0.f, 0.f, 0.f};
     for (int pi = tile.piece_begin; pi < tile.piece_end; ++pi) {
-        const SbPiece pc = a.pieces[pi];
+        // (in scalar registers the 512-thread kernel at N = 128 spills)
+        const SbPiece pc = WG <= 256 ? sb_kload(a.pieces, pi) : a.pieces[pi];
         if (pc.kind != SB_PIECE_MFMA) continue;          // never built into an MFMA tile
-        __syncthreads();                               // previous piece done with xrow and B
-        sb_expand_xrow_mfma(a.xr, pc.xr_begin, pc.xr_end, pc.ncols, xrow);
-        __syncthreads();
         sb_mfma_kloop<WG, NRHS, SPLIT, NU>(a, mb, pc, umi, N, n0, nt, xrow, B, acc);
     }
     const bool split = tile.ksplit > 1;
@@ -534,7 +539,7 @@ __device__ __forceinline__ void sb_spmm_mfma_tile(const SbSpmmArgs &a, int v, in
         n0 = k % NG * Cfg::NMAX;
     }
     const int nt = NRHS ? Cfg::NTMAX : N >> 4;
-    const SbTile tile = a.tiles[t];
+    const SbTile tile = sb_kload(a.tiles, __builtin_amdgcn_readfirstlane(t));
     const int mt = (tile.nrows + 15) >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int mine = mt > wave ? (mt - wave + NW - 1) / NW : 0;   // units of this wavefront (round robin)
