@@ -42,8 +42,13 @@ SablePlanOpts normalize_opts(const SablePlanOpts *in)
     // threads, 50 with 256 KiB, 37 with 128 KiB, 36 with 64 KiB; 64 matrices,
     // 336 MB, 91, 72, 75 and 78 us.  With 128 threads 61 us from 256 KiB to
     // 128 KiB, 45 with 64 KiB; with 64 threads 65 with 128 KiB, 37 with 32.
+    // SpMM: MFMA tiles at N = 16 256 KiB (20,011 rows 31.2 -> 27.6 us, 50,000
+    // rows 55.8 -> 54.3); at N = 32 half the tile took the 50,000 rows from
+    // 65 to 72 us.
     if (o.tile_bytes <= 0)
-        o.tile_bytes = o.op == SABLE_OP_SPMV ? 512 * (int64_t)std::min(std::max(o.wg, 64), 256) : 512 * 1024;
+        o.tile_bytes = o.op == SABLE_OP_SPMV ? 512 * (int64_t)std::min(std::max(o.wg, 64), 256)
+                       : o.n_rhs <= 16              ? 256 * 1024
+                                                    : 512 * 1024;
     if (o.max_seg_rows <= 0) o.max_seg_rows = o.wg;
     if (o.min_seg_rows <= 0) o.min_seg_rows = (o.op == SABLE_OP_SPMV) ? 8 : 16;
     if (o.mode < 0 || o.mode > 2) o.mode = SABLE_MODE_GRID;

@@ -93,7 +93,7 @@ typedef __attribute__((ext_vector_type(4))) float sb_f32x4;
 // lane, accumulators included), so two 256-thread workgroups share a CU, or
 // three
 #ifndef SB_MFMA_WAVES
-#define SB_MFMA_WAVES (SB_MFMA_THREE ? 3 : 2)
+#define SB_MFMA_WAVES (SB_MFMA_THREE || (SB_NRHS == 16 && SB_WG >= 256) ? 3 : 2)
 #endif
 
 __device__ __forceinline__ sb_bf16x8 sb_as_bf16x8(sb_u4 v) { return __builtin_bit_cast(sb_bf16x8, v); }
@@ -571,13 +571,186 @@ __device__ __forceinline__ void sb_spmm_mfma_tile(const SbSpmmArgs &a, int v, in
     }
 }
 
+// N = 16 and 32: the wavefronts share the k-steps instead of the rows.  A
+// k-step's X unit of a lane (8 rows, one column) is the lane's own B fragment
+// then, so X goes from L2 to registers and is split there: no staging through
+// LDS and no barrier per k-step, where at these N one or two wavefronts staged
+// X while the others waited (prefetch depths of 1 to 4 k-steps made no
+// difference; the staging wavefront's issue was the bound).  Every wavefront
+// holds all units of the pass, NU of them, and takes k-steps wave, wave + NW,
+// ...; the next one's A and X are in flight while one is multiplied.  At the
+// end the wavefronts' sums are added through LDS in wavefront order.
+//
+// For 256 threads and more.  At 20,011 rows and N = 16 with 256 threads both
+// launches took 36.5 us (cold 45.3) with the rows shared and 30.8 (41.1) so;
+// a batch of 16 matrices 77 us either way.  With 128 threads there are two
+// wavefronts to share the k-steps, and the batch's tiles have one or two:
+// 72 us with the rows shared, 76 so.
+#define SB_MFMA_KSPLIT(WG, N) ((WG) >= 256 && ((N) == 16 || (N) == 32))
+template <int WG, int NRHS>
+struct SbMfmaKs {
+    static constexpr int NW = WG / 64;
+    static constexpr int NT = NRHS / 16;
+    static constexpr int UN = 8;                            // units of a pass at most
+    static constexpr int G = NW <= 4 ? NW : 2;              // units summed at a time
+    static constexpr int SMEM_BYTES = NW * G * NT * 1024;
+};
+
+template <int WG, int NRHS, int SPLIT, int NU>
+__device__ __forceinline__ void sb_mfma_ksplit_pass(const SbSpmmArgs &a, const SbMatBufs &mb, const SbTile &tile,
+                                                    int u0, int nu, int mt, int *xrow, sb_f32x4 *red)
+{
+    using Ks = SbMfmaKs<WG, NRHS>;
+    using Pt = SbPasses<SPLIT>;
+    constexpr int NW = Ks::NW, NT = Ks::NT, G = Ks::G;
+    // k-steps of A and X ahead: what the units leave of the registers
+    constexpr int D = NU <= 4 ? 2 : 1;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int nb = lane & 15, kg = lane >> 4;
+    const sb_gfloat gX = (sb_gfloat)mb.x;
+    sb_f32x4 acc[NU][NT];
+#pragma unroll
+    for (int i = 0; i < NU; ++i)
+#pragma unroll
+        for (int t = 0; t < NT; ++t) acc[i][t] = sb_f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int pi = tile.piece_begin; pi < tile.piece_end; ++pi) {
+        const SbPiece pc = sb_kload(a.pieces, pi);
+        if (pc.kind != SB_PIECE_MFMA) continue;          // never built into an MFMA tile
+        const int K = pc.ksteps;
+        const SB_G sb_f4 *__restrict__ A = reinterpret_cast<const SB_G sb_f4 *>(sb_gp(mb.dval) + pc.data_off);
+        sb_f4 ar[D][NU][2];
+        // a unit past the last one repeats it (its sums are not stored)
+        auto load_a = [&](int sl, int i, int k) {
+            const int off = ((u0 + (i < nu ? i : nu - 1)) * K + k) * 128 + lane;
+            ar[sl][i][0] = __builtin_nontemporal_load(&A[off]);
+            ar[sl][i][1] = __builtin_nontemporal_load(&A[off + 64]);
+        };
+        auto clampk = [&](int k) { return k < K ? k : K - 1; };
+#pragma unroll
+        for (int sl = 0; sl < D; ++sl)
+#pragma unroll
+            for (int i = 0; i < NU; ++i) load_a(sl, i, clampk(wave + sl * NW));
+        __syncthreads();                                 // previous piece done with xrow
+        sb_expand_xrow_mfma(a.xr, pc.xr_begin, pc.xr_end, pc.ncols, xrow);
+        __syncthreads();
+        float xf[D][NT][8];
+        auto fetch_x = [&](int sl, int k) {
+            const int4 ra = *reinterpret_cast<const int4 *>(xrow + k * 32 + kg * 8);
+            const int4 rb = *reinterpret_cast<const int4 *>(xrow + k * 32 + kg * 8 + 4);
+            const int rows[8] = {ra.x, ra.y, ra.z, ra.w, rb.x, rb.y, rb.z, rb.w};
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+#pragma unroll
+                for (int j = 0; j < 8; ++j)
+                    xf[sl][t][j] = gX[(uint32_t)rows[j] * (uint32_t)NRHS + (uint32_t)(t * 16 + nb)];
+        };
+#pragma unroll
+        for (int sl = 0; sl < D; ++sl) fetch_x(sl, clampk(wave + sl * NW));
+        // D k-steps per trip; every load is unconditional (past the piece it
+        // reads the last k-step), so the waits stay exact
+        for (int k0 = wave; k0 < K; k0 += NW * D) {
+#pragma unroll
+            for (int sl = 0; sl < D; ++sl) {
+                const int ks = k0 + sl * NW;
+                const bool live = sl == 0 || ks < K;
+                sb_bf16x8 bt[NT][SPLIT];
+                if (live)
+#pragma unroll
+                    for (int t = 0; t < NT; ++t) {
+                        float v[8];
+#pragma unroll
+                        for (int j = 0; j < 8; ++j) v[j] = ks * 32 + kg * 8 + j < pc.ncols ? xf[sl][t][j] : 0.f;
+                        sb_split8<SPLIT>(v, bt[t]);
+                    }
+                fetch_x(sl, clampk(ks + D * NW));
+#pragma unroll
+                for (int i = 0; i < NU; ++i) {
+                    sb_bf16x8 at[SPLIT];
+                    if (live) {
+                        const float af[8] = {ar[sl][i][0].x, ar[sl][i][0].y, ar[sl][i][0].z, ar[sl][i][0].w,
+                                             ar[sl][i][1].x, ar[sl][i][1].y, ar[sl][i][1].z, ar[sl][i][1].w};
+                        sb_split8<SPLIT>(af, at);
+                    }
+                    load_a(sl, i, clampk(ks + D * NW));
+                    if (live)
+#pragma unroll
+                        for (int p = 0; p < Pt::N; ++p)
+#pragma unroll
+                            for (int t = 0; t < NT; ++t)
+                                acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(at[Pt::a(p)], bt[t][Pt::b(p)],
+                                                                                    acc[i][t], 0, 0, 0);
+                }
+            }
+        }
+    }
+    const bool split = tile.ksplit > 1;
+#pragma unroll
+    for (int i0 = 0; i0 < NU; i0 += G) {
+        if (i0 >= nu) break;
+        __syncthreads();                                 // red free
+#pragma unroll
+        for (int g = 0; g < G; ++g)
+            if (i0 + g < NU)
+#pragma unroll
+                for (int t = 0; t < NT; ++t) red[((wave * G + g) * NT + t) * 64 + lane] = acc[i0 + g][t];
+        __syncthreads();
+        const int u = u0 + i0 + wave;                    // wavefront g < G sums and stores unit i0 + g
+        if (wave >= G || i0 + wave >= nu) continue;
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+            sb_f32x4 s = red[(wave * NT + t) * 64 + lane];
+#pragma unroll
+            for (int w = 1; w < NW; ++w) s += red[((w * G + wave) * NT + t) * 64 + lane];
+            if (split) {
+                const int64_t blk = (int64_t)tile.part_blk + (int64_t)(tile.kpart * mt + u) * NT + t;
+                reinterpret_cast<SB_G sb_f32x4 *>(sb_gp(mb.part))[blk * 64 + lane] = s;
+            } else {
+                const int rbase = u * 16 + 4 * kg;
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (rbase + r < tile.nrows) sb_gp(mb.y)[(size_t)(tile.row0 + rbase + r) * NRHS + t * 16 + nb] = s[r];
+            }
+        }
+    }
+}
+
+// One MFMA work item at N = 16 or 32.
+template <int WG, int NRHS, int SPLIT>
+__device__ __forceinline__ void sb_mfma_ksplit_tile(const SbSpmmArgs &a, int t, int *xrow, unsigned char *smem)
+{
+    const SbTile tile = sb_kload(a.tiles, __builtin_amdgcn_readfirstlane(t));
+    const SbMatBufs mb = a.mats ? sb_kload(a.mats, tile.mat) : sb_mat_bufs(a, 0, nullptr);
+    const int mt = (tile.nrows + 15) >> 4;
+    sb_f32x4 *red = reinterpret_cast<sb_f32x4 *>(smem);
+    for (int u0 = 0; u0 < mt; u0 += SbMfmaKs<WG, NRHS>::UN) {
+        const int nu = mt - u0;
+        if (nu == 1)
+            sb_mfma_ksplit_pass<WG, NRHS, SPLIT, 1>(a, mb, tile, u0, nu, mt, xrow, red);
+        else if (nu == 2)
+            sb_mfma_ksplit_pass<WG, NRHS, SPLIT, 2>(a, mb, tile, u0, nu, mt, xrow, red);
+        else if (nu <= 4)
+            sb_mfma_ksplit_pass<WG, NRHS, SPLIT, 4>(a, mb, tile, u0, nu, mt, xrow, red);
+        else if (nu <= 6)
+            sb_mfma_ksplit_pass<WG, NRHS, SPLIT, 6>(a, mb, tile, u0, nu, mt, xrow, red);
+        else
+            sb_mfma_ksplit_pass<WG, NRHS, SPLIT, 8>(a, mb, tile, u0, nu < 8 ? nu : 8, mt, xrow, red);
+    }
+}
+
 template <int WG, int NRHS, int XCAP, int SPLIT>
 __device__ __forceinline__ void sb_spmm_mfma_body(const SbSpmmArgs &a)
 {
     using Cfg = SbMfmaCfg<WG, NRHS, SPLIT>;
+    constexpr bool KSPLIT = SB_MFMA_KSPLIT(WG, NRHS);
+    constexpr int SMEM = KSPLIT ? SbMfmaKs<WG, KSPLIT ? NRHS : 16>::SMEM_BYTES : Cfg::SMEM_BYTES;
     __shared__ __attribute__((aligned(16))) int xrow[XCAP + 32];   // k-steps read up to 31 past ncols
-    __shared__ __attribute__((aligned(16))) unsigned char smem[Cfg::SMEM_BYTES];
+    __shared__ __attribute__((aligned(16))) unsigned char smem[SMEM];
     __shared__ int next_tile;
-    sb_for_tiles(a.ntiles, a.mode, a.queue, &next_tile,
-                 [&](int t) { sb_spmm_mfma_tile<WG, NRHS, SPLIT>(a, t, xrow, smem); });
+    sb_for_tiles(a.ntiles, a.mode, a.queue, &next_tile, [&](int t) {
+        if constexpr (KSPLIT)
+            sb_mfma_ksplit_tile<WG, NRHS, SPLIT>(a, t, xrow, smem);
+        else
+            sb_spmm_mfma_tile<WG, NRHS, SPLIT>(a, t, xrow, smem);
+    });
 }
