@@ -660,7 +660,7 @@ size_t g_pinned_bytes = 0;
 
 struct PinnedBuf {
     PinnedBlock b{nullptr, 0};
-    int get(size_t bytes)
+    bool get(size_t bytes)
     {
         {
             std::lock_guard<std::mutex> lk(g_mu);
@@ -671,14 +671,18 @@ struct PinnedBuf {
                 b = g_pinned[best];
                 g_pinned.erase(g_pinned.begin() + best);
                 g_pinned_bytes -= b.bytes;
-                return SABLE_OK;
+                return true;
             }
         }
         size_t want = 64 << 10;                  // a few sizes, so that blocks are found again
         while (want < bytes) want <<= 1;
-        HIPOK(hipHostMalloc(&b.p, want, hipHostMallocDefault));
+        if (hipHostMalloc(&b.p, want, hipHostMallocDefault) != hipSuccess) {
+            (void)hipGetLastError();             // the caller has another way
+            b.p = nullptr;
+            return false;
+        }
         b.bytes = want;
-        return SABLE_OK;
+        return true;
     }
     ~PinnedBuf()
     {
@@ -934,15 +938,16 @@ int sable_plan_export(const SablePlan *p, int which, void *dst, int64_t *bytes)
 // takes 33.  Up to SABLE_PINNED_ROWS each the pinned memory is small (8 MiB).
 #define SABLE_PINNED_ROWS (1 << 20)
 
-static int run_host_spmv(SablePlan *p, const float *x, float *y, int64_t nx, int64_t ny)
+static int run_host_spmv(SablePlan *p, const float *x, float *y, int64_t nx, int64_t ny, bool &taken)
 {
     const int64_t nxp = (nx + 15) & ~(int64_t)15;
+    PinnedBuf pinned;
+    taken = pinned.get((nxp + ny) * 4);
+    if (!taken) return SABLE_OK;                 // no pinned memory: the runtime's copies
     if (p->xtmp_n < nx) {
         HIPOK(hipMalloc((void **)&p->d_xtmp, nx * 4));
         p->xtmp_n = nx;
     }
-    PinnedBuf pinned;
-    CHECKRC(pinned.get((nxp + ny) * 4));
     float *hx = (float *)pinned.b.p, *hy = hx + nxp;
     memcpy(hx, x, nx * 4);
     hipLaunchKernelGGL(sb_copy_words, dim3((unsigned)((nx + 255) / 256)), dim3(256), 0, p->stream, hx, p->d_xtmp, nx);
@@ -962,8 +967,11 @@ static int run_op(SablePlan *p, const float *x, float *y, int flags, int64_t nx,
     const float *dx = x;
     float *dy = y;
     if (flags & SABLE_HOST_PTRS) {
-        if (p->host.op == SABLE_OP_SPMV && p->own_stream && nx <= SABLE_PINNED_ROWS && ny <= SABLE_PINNED_ROWS)
-            return run_host_spmv(p, x, y, nx, ny);
+        if (p->host.op == SABLE_OP_SPMV && p->own_stream && nx <= SABLE_PINNED_ROWS && ny <= SABLE_PINNED_ROWS) {
+            bool taken = false;
+            const int rc = run_host_spmv(p, x, y, nx, ny, taken);
+            if (taken) return rc;
+        }
         if (p->xtmp_n < nx) {
             if (p->d_xtmp) hipFree(p->d_xtmp);
             p->d_xtmp = nullptr;
