@@ -454,7 +454,8 @@ int build_for_slots(const SableVbr &v, const uint8_t *route, const SablePlanOpts
     }
     for (const double f : {1.6, 1.9, 2.2}) {
         if ((int64_t)P.tiles.size() <= slots || f * share > (double)o.tile_bytes) return SABLE_OK;
-        if (f * share <= 32.0 * 1024) continue;
+        // (a larger target leaves at best proportionally fewer tiles)
+        if (f * share <= 32.0 * 1024 || 1.4 * (double)P.tiles.size() > f * (double)slots) continue;
         target(f * share);
         HostPlan Q;
         rc = build_host_plan_once(v, route, oo, spans, Q, err);
