@@ -20,6 +20,7 @@
 #include <sstream>
 #include <string>
 #include <array>
+#include <type_traits>
 #include <vector>
 #include <sys/stat.h>
 #include <sys/time.h>
@@ -426,10 +427,12 @@ int upload(T **dptr, const std::vector<T> &v, int64_t &bytes)
 {
     *dptr = nullptr;
     if (v.empty()) return SABLE_OK;
-    // 256 bytes past the end: kernels read one entry past an array's last
-    // (an empty row's first entry) without using it
-    HIPOK(hipMalloc((void **)dptr, v.size() * sizeof(T) + 256));
-    HIPOK(hipMemcpy(*dptr, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice));
+    // 256 bytes past the end, zero for values: kernels read one entry past an
+    // array's last (an empty row's first entry) without using it
+    const size_t n = v.size() * sizeof(T);
+    HIPOK(hipMalloc((void **)dptr, n + 256));
+    if (std::is_same<T, float>::value) HIPOK(hipMemset((char *)*dptr + n, 0, 256));
+    HIPOK(hipMemcpy(*dptr, v.data(), n, hipMemcpyHostToDevice));
     bytes += (int64_t)(v.size() * sizeof(T));
     return SABLE_OK;
 }

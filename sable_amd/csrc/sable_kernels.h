@@ -587,9 +587,10 @@ __device__ __forceinline__ void sb_static_for(F f)
 // and X row) to the row's V columns at X + co: n entries of this lane's row
 // are valid (n may differ between the rows of a wavefront), most is the
 // largest n, least the smallest.  F entries' X rows are in flight at a time.
-// Where some row has run out, its entries repeat its last one and add
-// nothing (their X is taken as 0, so an infinity there stays out).  FAR: X is
-// 4 GiB or more.
+// Where some row has run out, its entries repeat its last X row and add
+// nothing: the caller gives the value 0 there and X is taken as 0, so neither
+// a value nor an X that is not finite gets into another entry's sum.  FAR: X
+// is 4 GiB or more.
 template <int BATCH, int F, int V, bool FAR>
 __device__ __forceinline__ void sb_f32_entries(const SB_G float *__restrict__ X, int N, uint32_t co, float val, int col,
                                                int n, int least, int most, float (&acc)[V])
@@ -770,8 +771,10 @@ __device__ __forceinline__ void sb_f32_task(const SbSpmmArgs &a, const SbTask &t
         for (int u = 0; u < U; ++u)
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
+                // past the row's end (an empty row's entry is not its own): 0
                 const int e = lo[u][q] + max(min(i, n[u][q] - 1), 0);
-                v0[u][q] = sv[e];
+                const float v = sv[e];
+                v0[u][q] = i < n[u][q] ? v : 0.f;
                 c0[u][q] = sc[e];
             }
 #pragma unroll
@@ -789,6 +792,7 @@ __device__ __forceinline__ void sb_f32_task(const SbSpmmArgs &a, const SbTask &t
                     if (e0 > 0) {
                         const int e = lo[u][q] + max(min(e0 + i, n[u][q] - 1), 0);
                         v = sv[e];
+                        v = e0 + i < n[u][q] ? v : 0.f;
                         c = n[u][q] > 0 ? sc[e] : 0;
                     }
                     sb_f32_entries<16, 4, T, FAR>(X, N, co, v, c, n[u][q] - e0, least - e0, most - e0, s);
@@ -858,8 +862,10 @@ __device__ __forceinline__ void sb_f32_sparse_task(const SbSpmmArgs &a, const Sb
         }
 #pragma unroll
         for (int k = 0; k < IT; ++k) {
+            // past the row's end (an empty row's entry is not its own): 0
             const int e = lo[k] + max(min(q, n[k] - 1), 0);
-            v0[k] = sv[e];
+            const float v = sv[e];
+            v0[k] = q < n[k] ? v : 0.f;
             c0[k] = sc[e];
         }
 #pragma unroll
@@ -874,7 +880,7 @@ __device__ __forceinline__ void sb_f32_sparse_task(const SbSpmmArgs &a, const Sb
                 const float vn = sv[e];
                 const int cn = sc[e];
                 sb_f32_entries<BATCH, F, 4, FAR>(X, N, co, v, c, n[k] - e0, least - e0, most - e0, s[k]);
-                v = vn;
+                v = e0 + BATCH + q < n[k] ? vn : 0.f;
                 c = n[k] > 0 ? cn : 0;
             }
         }
