@@ -1599,16 +1599,24 @@ int check_partition(const int64_t *part, int32_t nparts, int64_t n, const char *
     return SABLE_OK;
 }
 
-int scan_exclusive(int64_t *d_in, int64_t n, int64_t *d_out, DevBufs &b)
+int64_t scan_blocks(int64_t n) { return (n + SB_SCAN_BLOCK - 1) / SB_SCAN_BLOCK; }
+
+// d_tot: scan_blocks(n) totals
+int scan_exclusive_with(int64_t *d_in, int64_t n, int64_t *d_out, int64_t *d_tot)
 {
-    const int64_t nblk = (n + SB_SCAN_BLOCK - 1) / SB_SCAN_BLOCK;
-    int64_t *d_tot = nullptr;
-    CHECKRC(b.alloc((void **)&d_tot, nblk * sizeof(int64_t)));
+    const int64_t nblk = scan_blocks(n);
     hipLaunchKernelGGL(sb_scan_blocks, dim3((unsigned)nblk), dim3(SB_SCAN_BLOCK), 0, nullptr, d_in, n, d_out, d_tot);
     hipLaunchKernelGGL(sb_scan_totals, dim3(1), dim3(SB_SCAN_BLOCK), 0, nullptr, d_tot, nblk);
     hipLaunchKernelGGL(sb_scan_add, dim3((unsigned)nblk), dim3(SB_SCAN_BLOCK), 0, nullptr, d_out, n, d_tot);
     HIPOK(hipGetLastError());
     return SABLE_OK;
+}
+
+int scan_exclusive(int64_t *d_in, int64_t n, int64_t *d_out, DevBufs &b)
+{
+    int64_t *d_tot = nullptr;
+    CHECKRC(b.alloc((void **)&d_tot, scan_blocks(n) * sizeof(int64_t)));
+    return scan_exclusive_with(d_in, n, d_out, d_tot);
 }
 
 }  // namespace
@@ -1642,7 +1650,7 @@ extern "C" int sable_partition_cuts(const int64_t *indptr, const int32_t *indice
     const int64_t o_ip = carve((ncols + 1) * 8), o_ix = carve(nnz * 4), o_v = carve(nnz * 8), o_tip = carve((nrows + 1) * 8),
                   o_tix = carve(nnz * 4), o_tv = carve(nnz * 8), o_cnt = carve(nchunk * nrows * 4),
                   o_tot = carve((nrows + 1) * 8), o_cs = carve(ncols * 8), o_rs = carve(nrows * 8), o_cc = carve(ncols + 1),
-                  o_rc = carve(nrows + 1), o_bad = carve(4);
+                  o_rc = carve(nrows + 1), o_bad = carve(4), o_st = carve(scan_blocks(nrows + 1) * 8);
     DevBufs b;
     char *m = nullptr;
     CHECKRC(b.alloc((void **)&m, at));
@@ -1677,10 +1685,14 @@ extern "C" int sable_partition_cuts(const int64_t *indptr, const int32_t *indice
     hipLaunchKernelGGL(sb_zero_i32, dim3(2048), dim3(256), 0, nullptr, cnt, nchunk * nrows);
     hipLaunchKernelGGL(sb_count_rows, dim3((unsigned)nchunk), dim3(1024), 0, nullptr, ip, ix, nrows, ncols, per, cnt);
     hipLaunchKernelGGL(sb_prefix_rows, dim3((unsigned)((nrows + 256) / 256)), dim3(256), 0, nullptr, cnt, nrows, nchunk, tot);
-    const int sc = scan_exclusive(tot, nrows + 1, tip, b);
-    hipLaunchKernelGGL(sb_place_rows, dim3((unsigned)nchunk), dim3(512), 0, nullptr, ip, ix, v, nrows, ncols, per, cnt, tip,
-                       tix, tv);
-    axis(tip, tix, tv, nrows, ncols, rs, rc);
+    // the placing kernel writes where the scan says: only after all of its
+    // launches went out (its scratch is carved above, so none fails for memory)
+    const int sc = scan_exclusive_with(tot, nrows + 1, tip, (int64_t *)(m + o_st));
+    if (sc == SABLE_OK) {
+        hipLaunchKernelGGL(sb_place_rows, dim3((unsigned)nchunk), dim3(512), 0, nullptr, ip, ix, v, nrows, ncols, per, cnt,
+                           tip, tix, tv);
+        axis(tip, tix, tv, nrows, ncols, rs, rc);
+    }
     hipEventRecord(e1, nullptr);
     const hipError_t le = hipGetLastError();
     const hipError_t se = hipEventSynchronize(e1);
