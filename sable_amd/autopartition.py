@@ -170,17 +170,34 @@ def _axis_cuts_gpu(M, threshold, similarity, return_sim=False):
     return (cuts, sim[:max(n - 1, 0)]) if return_sim else cuts
 
 
+def _device_transpose_pays(nrows, ncols, nnz):
+    """Whether the GPU's transpose beats the host's.  A workgroup places the
+    columns of its chunk one after another, about 0.35 us each, and there are
+    at most 512 chunks, fewer where their counts would pass 64 MiB (one chunk
+    from 8.4 M rows); the host transpose and the second upload take about
+    6 ns per entry.  Both axes, GPU against host transpose: 0.44 and 0.72 ms
+    at 20,000 lines of 5 entries, 1.6 and 2.8 at 100,000, 9.8 and 13.8 at
+    500,000, 31.8 and 31.6 at 1,000,000; 1.1 and 13.9 ms at 6,000 lines of
+    300.  A chunk of 4,096 columns is 1.4 ms at most."""
+    chunks = min(512, ncols, max(1, (16 << 20) // nrows))
+    per_chunk = -(-ncols // chunks)
+    return per_chunk <= 4096 or 64 * per_chunk <= nnz
+
+
 def _both_cuts_gpu(A, threshold, similarity):
     """Both axes from one upload of the CSC matrix A, transposed on the GPU
     (sable_partition_cuts), or None for a matrix this does not take: values
     that are not real, columns whose rows are not strictly ascending
     (duplicates are summed and rows sorted by the per-axis path), more than
-    2^25 lines, or more memory than is free.  The host transpose took a third
-    of a conversion's time."""
+    2^25 lines, more memory than is free, or so many lines for its entries
+    that the host's transpose is faster.  The host transpose took a third of a
+    conversion's time."""
     from . import runtime
     from ._lib import lib, check, SableError, SABLE_ERR_OOM, SABLE_ERR_UNSUPPORTED
     kind = _GPU_KIND.get(similarity)
     if kind is None or A.dtype.kind not in "fiub" or min(A.shape) == 0 or max(A.shape) > 1 << 25:
+        return None
+    if not _device_transpose_pays(A.shape[0], A.shape[1], int(A.indptr[-1])):
         return None
     ip = np.ascontiguousarray(A.indptr, dtype=np.int64)
     ix = np.ascontiguousarray(A.indices[:ip[-1]], dtype=np.int32)
