@@ -658,6 +658,8 @@ struct PinnedBlock {
     void *p;
     size_t bytes;
 };
+// (a lock of its own: g_mu is held while a kernel compiles)
+std::mutex g_pinned_mu;
 std::vector<PinnedBlock> g_pinned;
 size_t g_pinned_bytes = 0;
 
@@ -666,7 +668,7 @@ struct PinnedBuf {
     bool get(size_t bytes)
     {
         {
-            std::lock_guard<std::mutex> lk(g_mu);
+            std::lock_guard<std::mutex> lk(g_pinned_mu);
             size_t best = g_pinned.size();
             for (size_t i = 0; i < g_pinned.size(); ++i)
                 if (g_pinned[i].bytes >= bytes && (best == g_pinned.size() || g_pinned[i].bytes < g_pinned[best].bytes)) best = i;
@@ -691,7 +693,7 @@ struct PinnedBuf {
     {
         if (!b.p) return;
         {
-            std::lock_guard<std::mutex> lk(g_mu);
+            std::lock_guard<std::mutex> lk(g_pinned_mu);
             if (g_pinned_bytes + b.bytes <= SABLE_PINNED_KEPT) {
                 g_pinned.push_back(b);
                 g_pinned_bytes += b.bytes;
