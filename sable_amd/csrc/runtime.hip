@@ -1891,6 +1891,9 @@ int compress_on_device(const double *d_val, const int64_t *d_indx, const int64_t
     }
     h->nval2 = h->indx2.back();
     h->nub = (int64_t)h->ublocks.size();
+    int64_t sparse_heights = 0;
+    for (int32_t a = 0; a < nbr; ++a)
+        for (int64_t k = std::max<int64_t>(bpntrb[a], 0); k < bpntre[a]; ++k) sparse_heights += sp[k] ? rpntr[a + 1] - rpntr[a] : 0;
     DevBufs b;
     int64_t *d_rp = nullptr, *d_cp = nullptr, *d_bb = nullptr, *d_be = nullptr, *d_dblk = nullptr,
             *d_indx2 = nullptr, *d_cnt = nullptr;
@@ -1926,16 +1929,26 @@ int compress_on_device(const double *d_val, const int64_t *d_indx, const int64_t
         hipLaunchKernelGGL(sb_gather_dense, dim3((unsigned)((ndense * parts + 3) / 4)), dim3(256), 0, nullptr, d_val,
                            d_indx, d_dblk, d_indx2, ndense, parts, h->d_val2);
     }
-    // values of sparse blocks per row: the columns a row's threads walk
-    const int64_t mean = (indx[nblocks] - h->nval2) / nrows;
-    const int segs = (int)std::min<int64_t>(std::max<int64_t>(mean / SB_CSR_COLS, 1), SB_CSR_SEGS);
-    const dim3 csr_grid((unsigned)((nrows + 63) / 64)), csr_block(64 * segs);
+    // values of sparse blocks per row: the columns a row's threads walk; and
+    // per row of a sparse block: their mean width
+    const int64_t sparse_values = indx[nblocks] - h->nval2;
+    const int64_t mean = sparse_values / nrows;
+    const bool wide = sparse_values >= SB_CSR_WIDTH * sparse_heights;
+    const int segs = wide ? (int)std::min<int64_t>(std::max<int64_t>(mean / SB_CSR_COLS, 1), SB_CSR_SEGS) : 1;
+    auto csr_rows = [&](int64_t *rowptr, int64_t *cols, double *vals) {
+        if (segs > 1)
+            hipLaunchKernelGGL(sb_csr_rows<true>, dim3((unsigned)((nrows + 63) / 64)), dim3(64 * segs), 0, nullptr, d_val,
+                               d_indx, d_bindx, d_rp, d_cp, d_bb, d_be, d_sp, d_rmap, nrows, ncols, d_cnt, rowptr, cols,
+                               vals, d_last);
+        else
+            hipLaunchKernelGGL(sb_csr_rows<false>, g256(nrows), dim3(256), 0, nullptr, d_val, d_indx, d_bindx, d_rp, d_cp,
+                               d_bb, d_be, d_sp, d_rmap, nrows, ncols, d_cnt, rowptr, cols, vals, d_last);
+    };
     int64_t nnz = 0;
     if (h->nub > 0) {
         hipLaunchKernelGGL(sb_part_map, g256(nrows), dim3(256), 0, nullptr, d_rp, nbr, nrows, d_rmap);
         HIPOK(hipMemsetAsync(d_last, 0, sizeof(int32_t), nullptr));
-        hipLaunchKernelGGL(sb_csr_rows, csr_grid, csr_block, 0, nullptr, d_val, d_indx, d_bindx, d_rp, d_cp,
-                           d_bb, d_be, d_sp, d_rmap, nrows, ncols, d_cnt, nullptr, nullptr, nullptr, d_last);
+        csr_rows(nullptr, nullptr, nullptr);
         HIPOK(hipMalloc((void **)&h->d_rowptr, (nrows + 1) * sizeof(int64_t)));
         CHECKRC(scan_exclusive(d_cnt, nrows, h->d_rowptr, b));
         int64_t lastptr = 0, lastcnt = 0;
@@ -1951,9 +1964,7 @@ int compress_on_device(const double *d_val, const int64_t *d_indx, const int64_t
             h->nnz = nnz + (pad ? 1 : 0);
             HIPOK(hipMalloc((void **)&h->d_cols, h->nnz * sizeof(int64_t)));
             HIPOK(hipMalloc((void **)&h->d_vals, h->nnz * sizeof(double)));
-            hipLaunchKernelGGL(sb_csr_rows, csr_grid, csr_block, 0, nullptr, d_val, d_indx, d_bindx, d_rp, d_cp,
-                               d_bb, d_be, d_sp, d_rmap, nrows, ncols, d_cnt, h->d_rowptr, h->d_cols, h->d_vals,
-                               d_last);
+            csr_rows(h->d_rowptr, h->d_cols, h->d_vals);
             if (pad) {
                 const int64_t c = ncols - 1;
                 const double z = 0.0;

@@ -258,43 +258,54 @@ __global__ void __launch_bounds__(256) sb_gather_dense(const double *__restrict_
 
 // per row: the nonzero values of its sparse-routed blocks (count pass when
 // cols == nullptr, fill pass otherwise); lastcol is set when one of them is
-// in the last column.  A workgroup holds 64 consecutive rows, so a
+// in the last column.  SPLIT: a workgroup holds 64 consecutive rows, so a
 // wavefront's loads of a column are contiguous, and blockDim.x / 64 segments
-// of their columns.  Bound by each thread's chain of column loads: one
-// segment per 32 sparse columns of the mean row, up to SB_CSR_SEGS.  On the
-// same matrix (248 sparse blocks) the count took 222 us with a thread per row
-// and takes 124, the fill 250 and 179; shares of 8 columns measured the same
-// there (125, 173).
+// of their columns; else a thread walks its row alone.  Bound by each thread's
+// chain of column loads: one segment per 32 sparse columns of the mean row, up
+// to SB_CSR_SEGS.  On the same matrix (248 sparse blocks) the count took
+// 222 us with a thread per row and takes 124, the fill 250 and 179; shares of 8
+// columns measured the same there (125, 173).
+// Every segment walks the row's block list and the fill counts before it
+// writes, so blocks of fewer than SB_CSR_WIDTH columns in the mean are not
+// split.  Both passes and the scan, 20,000 rows of 256 sparse columns, alone
+// and split: 2 columns a block 541 and 697 us, 4 377 and 332, 8 272 and 231,
+// 16 241 and 181, 100 182 and 150; 30 blocks of one column a row, with the
+// fill counting, 339, without 266 (40,000 rows).
 #define SB_CSR_SEGS 16
 #define SB_CSR_COLS 32
+#define SB_CSR_WIDTH 4
 
-__global__ void __launch_bounds__(64 * SB_CSR_SEGS)
+template <bool SPLIT>
+__global__ void __launch_bounds__(SPLIT ? 64 * SB_CSR_SEGS : 256)
 sb_csr_rows(const double *__restrict__ val, const int64_t *__restrict__ indx, const int64_t *__restrict__ bindx,
             const int64_t *__restrict__ rpntr, const int64_t *__restrict__ cpntr, const int64_t *__restrict__ bpntrb,
             const int64_t *__restrict__ bpntre, const uint8_t *__restrict__ sparse, const int32_t *__restrict__ rmap,
             int64_t nrows, int64_t ncols, int64_t *__restrict__ cnt, const int64_t *__restrict__ rowptr,
             int64_t *__restrict__ cols, double *__restrict__ vals, int32_t *__restrict__ lastcol)
 {
-    __shared__ int64_t part[SB_CSR_SEGS][64];
-    const int lane = (int)(threadIdx.x & 63), seg = (int)(threadIdx.x >> 6), segs = (int)(blockDim.x >> 6);
-    const int64_t r = (int64_t)blockIdx.x * 64 + lane;
+    const int lane = (int)(threadIdx.x & 63), seg = SPLIT ? (int)(threadIdx.x >> 6) : 0;
+    const int segs = SPLIT ? (int)(blockDim.x >> 6) : 1;
+    const int64_t r = SPLIT ? (int64_t)blockIdx.x * 64 + lane : (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const bool live = r < nrows;
     const int64_t a = live ? rmap[r] : 0;
     const int64_t kb = live && bpntrb[a] >= 0 ? bpntrb[a] : 0, ke = live && bpntrb[a] >= 0 ? bpntre[a] : 0;
     const int64_t h = live ? rpntr[a + 1] - rpntr[a] : 0, lr = live ? r - rpntr[a] : 0;
     // columns of the row's sparse blocks, and this segment's part of them
-    int64_t total = 0;
-    for (int64_t k = kb; k < ke; ++k)
-        if (sparse[k]) total += cpntr[bindx[k] + 1] - cpntr[bindx[k]];
-    const int64_t s0 = total * seg / segs, s1 = total * (seg + 1) / segs;
+    int64_t s0 = 0, s1 = INT64_MAX;
+    if (SPLIT) {
+        int64_t total = 0;
+        for (int64_t k = kb; k < ke; ++k)
+            if (sparse[k]) total += cpntr[bindx[k] + 1] - cpntr[bindx[k]];
+        s0 = total * seg / segs, s1 = total * (seg + 1) / segs;
+    }
     // calls f(column, value) for the segment's nonzero values in order
     auto walk = [&](auto f) {
         int64_t at = 0;
         for (int64_t k = kb; k < ke && at < s1; ++k) {
             if (!sparse[k]) continue;
             const int64_t b = bindx[k], c0 = cpntr[b], w = cpntr[b + 1] - c0;
-            const int64_t from = s0 > at ? s0 - at : 0, to = s1 - at < w ? s1 - at : w;
-            at += w;
+            const int64_t from = SPLIT && s0 > at ? s0 - at : 0, to = SPLIT && s1 - at < w ? s1 - at : w;
+            at += SPLIT ? w : 0;
             const double *__restrict__ blk = val + indx[k] + lr;
             // eight columns per step, their loads issued together (a
             // column past the part reads its last column again)
@@ -308,24 +319,26 @@ sb_csr_rows(const double *__restrict__ val, const int64_t *__restrict__ indx, co
             }
         }
     };
-    int64_t n = 0;
-    walk([&](int64_t c, double) {
-        ++n;
-        if (!cols && c == ncols - 1) *lastcol = 1;
-    });
-    part[seg][lane] = n;
-    __syncthreads();
+    int64_t n = 0, before = 0;
+    if (!cols || SPLIT)
+        walk([&](int64_t c, double) {
+            ++n;
+            if (!cols && c == ncols - 1) *lastcol = 1;
+        });
+    if (SPLIT) {
+        __shared__ int64_t part[SB_CSR_SEGS][64];
+        part[seg][lane] = n;
+        __syncthreads();
+        // the segments before this one (fill), all of them (count)
+        for (int q = 0; q < (cols ? seg : segs); ++q) before += part[q][lane];
+        n = before;
+    }
     if (!live) return;
     if (!cols) {
-        if (seg == 0) {
-            int64_t s = 0;
-            for (int q = 0; q < segs; ++q) s += part[q][lane];
-            cnt[r] = s;
-        }
+        if (seg == 0) cnt[r] = n;
         return;
     }
-    int64_t pos = rowptr[r];
-    for (int q = 0; q < seg; ++q) pos += part[q][lane];
+    int64_t pos = rowptr[r] + before;
     walk([&](int64_t c, double x) {
         cols[pos] = c;
         vals[pos] = x;
