@@ -83,6 +83,9 @@ PRECOMPILE = [
 ] + [
     (k, 256, 4, xcap, n, 8) for k in (2, 3) for n in (16, 32, 64, 128, 256) for xcap in (256, 512, 1024, 2048)
 ] + [
+    (k, wg, 4, 256, n, 8) for k, wg, n in ((2, 128, 96), (2, 256, 96), (3, 256, 96), (2, 256, 144), (2, 128, 160),
+                                           (2, 256, 160), (2, 256, 224), (2, 256, 240))
+] + [
     (k, 512, 4, xcap, n, 8) for k in (2, 3) for n in (16, 128) for xcap in (512, 1024, 2048)
 ] + [
     # the 256-matrix batch's SpMM members (N = 16, 128-thread workgroups)

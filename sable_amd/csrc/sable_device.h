@@ -113,7 +113,12 @@ struct SbTask {
 // threads, whose registers and LDS then leave room for two or three of them
 // on a compute unit, all of N in larger ones.  On the 50,000-row SpMM at
 // N = 128 (dense blocks alone) 64-column workgroups of 256 threads took
-// 88 us and full-width ones 107 us; at 512 threads 100 us and 84 us.
+// 88 us and full-width ones 107 us; at 512 threads 100 us and 84 us.  Widths
+// that are no multiple of 64 take groups of 48 or 32: the full-width kernels
+// spill (500 to 1,300 bytes a lane above N = 144).  A 3,001-row matrix of
+// dense blocks, full width and in groups, us: N = 96 43.7 and 24.1, N = 144
+// 74.7 and 25.4, N = 160 74.8 and 26.9 (128 threads: 51 and 30, 102 and 31,
+// 124 and 21); N = 224 31.0 and N = 240 34.2 in groups, N = 192 in 64s 24.0.
 // A wavefront holds two 16-row units across the columns (their FP32
 // accumulators plus the double-buffered A fragments), which bounds a tile at
 // SB_MFMA_MAX_ROWS(N, WG) rows (and 256).
