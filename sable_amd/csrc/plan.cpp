@@ -816,10 +816,12 @@ int build_host_plan_once(const SableVbr &v, const uint8_t *route, const SablePla
             return st;
         };
         auto vec_segments = [&](double work_v) {
+            // SpMM: whole 16-row fragments of the matrix instructions, where
+            // the limit holds one
+            if (spmm && max_rows >= 16) return cut(((h + 15) / 16 + max_rows / 16 - 1) / (max_rows / 16), true);
             int64_t nseg = (h + max_rows - 1) / max_rows;
             const int64_t want = spmm ? 1 : (int64_t)std::ceil(work_v / (double)o.tile_bytes);
-            // SpMM: whole 16-row fragments of the matrix instructions
-            return cut(std::max<int64_t>(nseg, std::min<int64_t>(want, (h + min_rows - 1) / min_rows)), spmm);
+            return cut(std::max<int64_t>(nseg, std::min<int64_t>(want, (h + min_rows - 1) / min_rows)), false);
         };
         if (spmm && !mgroups.empty()) {
             // MFMA tiles (first launch): tall, multiples of 16 rows, only the
