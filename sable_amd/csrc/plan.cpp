@@ -385,8 +385,30 @@ double emit_wave_slices(HostPlan &P, SablePlanStats &S, SbTile &t, const std::ve
 }
 
 namespace {
+// What the tiles of an SpMV plan follow from besides the options: the rows
+// and the value bytes of every block row or row span.
+struct Survey {
+    struct Span {
+        int32_t h;
+        double work;
+    };
+    std::vector<Span> spans;
+    int64_t bytes = 0;        // 4 per dense value, 6 per sparse entry
+};
+
+// The plan, or with a survey only that.
 int build_host_plan_once(const SableVbr &v, const uint8_t *route, const SablePlanOpts &o, bool spans, HostPlan &P,
-                         std::string &err);
+                         std::string &err, Survey *survey = nullptr);
+
+// SpMV: the tiles a block row or row span of h rows is cut into.
+int64_t spmv_segments(const SablePlanOpts &o, int32_t h, double work)
+{
+    const int64_t max_rows = std::max(std::min(o.max_seg_rows, o.wg), 1);
+    const int64_t min_rows = std::max<int64_t>(1, std::min<int64_t>(o.min_seg_rows, max_rows));
+    const int64_t nseg = (h + max_rows - 1) / max_rows;
+    const int64_t want = (int64_t)std::ceil(work / (double)o.tile_bytes);
+    return std::min<int64_t>(std::max(nseg, std::min(want, (h + min_rows - 1) / min_rows)), h);
+}
 
 // min_tiles asked for: the tile target is halved until there are that many
 // tiles (or tiles are 16 KiB).
@@ -423,49 +445,35 @@ int build_with_min_tiles(const SableVbr &v, const uint8_t *route, const SablePla
 int build_for_slots(const SableVbr &v, const uint8_t *route, const SablePlanOpts &o, bool spans, HostPlan &P,
                     std::string &err)
 {
-    int rc = validate_vbr(v, err);
+    Survey survey;
+    const int rc = build_host_plan_once(v, route, o, spans, P, err, &survey);
     if (rc) return rc;
     const int64_t slots = std::max<int64_t>(1, (int64_t)SB_SIMDS * std::max(2, SB_SPMV_WAVES(o.unroll)) * 64 / o.wg);
-    // value bytes of the plan: 4 per dense value, 6 per sparse entry
-    int64_t bytes = 0;
-    for (int64_t k = 0; k < v.nblocks; ++k) {
-        const float *b = v.val + v.indx[k];
-        const int64_t n = v.indx[k + 1] - v.indx[k];
-        if (route && route[k] == SABLE_ROUTE_SPARSE) {
-            int64_t c = 0;
-            for (int64_t e = 0; e < n; ++e) c += b[e] != 0.f;
-            bytes += 6 * c;
-        } else {
-            bytes += 4 * n;
-        }
-    }
-    const double share = (double)bytes / (double)slots;
-    SablePlanOpts oo = o;
-    auto target = [&](double bytes) {
+    const double share = (double)survey.bytes / (double)slots;
+    auto with_target = [&](double bytes) {
+        SablePlanOpts oo = o;
         oo.tile_bytes = std::min<int64_t>(o.tile_bytes, std::max<int64_t>((int64_t)bytes, 32 * 1024));
-        return oo.tile_bytes;
+        return oo;
     };
-    target(1.4 * share);
-    rc = build_host_plan_once(v, route, oo, spans, P, err);
-    if (rc) return rc;
-    if ((int64_t)P.tiles.size() * 2 < SB_CUS && oo.tile_bytes == 32 * 1024) {
-        oo.tile_bytes = 16 * 1024;
-        return build_host_plan_once(v, route, oo, spans, P, err);
-    }
-    for (const double f : {1.6, 1.9, 2.2}) {
-        if ((int64_t)P.tiles.size() <= slots || f * share > (double)o.tile_bytes) return SABLE_OK;
-        // (a larger target leaves at best proportionally fewer tiles)
-        if (f * share <= 32.0 * 1024 || 1.4 * (double)P.tiles.size() > f * (double)slots) continue;
-        target(f * share);
-        HostPlan Q;
-        rc = build_host_plan_once(v, route, oo, spans, Q, err);
-        if (rc) return rc;
-        if ((int64_t)Q.tiles.size() <= slots) {
-            P = std::move(Q);
-            return SABLE_OK;
+    auto tiles = [&](const SablePlanOpts &oo) {
+        int64_t n = 0;
+        for (auto &s : survey.spans) n += spmv_segments(oo, s.h, s.work);
+        return n;
+    };
+    SablePlanOpts best = with_target(1.4 * share);
+    const int64_t first = tiles(best);
+    if (first * 2 < SB_CUS && best.tile_bytes == 32 * 1024) {
+        best.tile_bytes = 16 * 1024;
+    } else {
+        for (const double f : {1.6, 1.9, 2.2}) {
+            if (first <= slots || f * share > (double)o.tile_bytes) break;
+            const SablePlanOpts oo = with_target(f * share);
+            if (tiles(oo) > slots) continue;
+            best = oo;
+            break;
         }
     }
-    return SABLE_OK;
+    return build_host_plan_once(v, route, best, spans, P, err);
 }
 }
 
@@ -488,7 +496,7 @@ int build_host_plan(const SableVbr &v, const uint8_t *route, const SablePlanOpts
 
 namespace {
 int build_host_plan_once(const SableVbr &v, const uint8_t *route, const SablePlanOpts &o, bool spans, HostPlan &P,
-                         std::string &err)
+                         std::string &err, Survey *survey)
 {
     int rc = validate_vbr(v, err);
     if (rc) return rc;
@@ -526,10 +534,9 @@ int build_host_plan_once(const SableVbr &v, const uint8_t *route, const SablePla
                               ? std::max(16, std::min(SB_MFMA_MAX_ROWS(o.n_rhs, o.wg), (o.max_seg_rows / 16) * 16))
                               : 16;
     max_rows = std::max(max_rows, 1);
-    const int min_rows = std::max(1, std::min(o.min_seg_rows, max_rows));
 
     // count nonzeros (plan-invariant flops basis)
-    for (int64_t i = 0; i < v.indx[v.nblocks]; ++i) S.nnz += (v.val[i] != 0.0f);
+    for (int64_t i = 0; !survey && i < v.indx[v.nblocks]; ++i) S.nnz += (v.val[i] != 0.0f);
 
     // SpMV: a run of consecutive short block rows (at most SB_SPMV_SHORT_ROWS
     // rows and SB_SPMV_SHORT_VALUES stored values each) is planned as one row
@@ -619,17 +626,23 @@ int build_host_plan_once(const SableVbr &v, const uint8_t *route, const SablePla
         auto mgroups = group_columns(mfma, v, mcap);
 
         // sparse entries of the row span (for costing)
-        int64_t sp_total = 0;
+        int64_t sp_total = 0, sp_kept = 0;
         for (int64_t k : sparse) {
             const float *bv = v.val + v.indx[k];
             const int64_t n = (int64_t)(v.cpntr[v.bindx[k] + 1] - v.cpntr[v.bindx[k]]) * geo.height(k);
-            if (geo.keeps(k)) sp_total += n;
+            if (geo.keeps(k)) sp_kept += n;
             else for (int64_t i = 0; i < n; ++i) sp_total += (bv[i] != 0.0f);
         }
+        sp_total += sp_kept;
         int64_t wd = 0, wm = 0;
         for (auto &g : dgroups) wd += group_width(g);
         for (auto &g : mgroups) wm += group_width(g);
         const double work = 4.0 * h * (double)(wd + wm) + 6.0 * sp_total + 4.0 * (h + 1) * sgroups.size();
+        if (survey) {
+            survey->spans.push_back({h, work});
+            survey->bytes += 4 * (int64_t)h * wd + 6 * sp_total - 2 * sp_kept;
+            continue;
+        }
 
         // Emits the tile of rows [s0, s0+hs) of this block row with the
         // pieces of the selected routes (vector routes: dense FP32 and
@@ -819,9 +832,7 @@ int build_host_plan_once(const SableVbr &v, const uint8_t *route, const SablePla
             // SpMM: whole 16-row fragments of the matrix instructions, where
             // the limit holds one
             if (spmm && max_rows >= 16) return cut(((h + 15) / 16 + max_rows / 16 - 1) / (max_rows / 16), true);
-            int64_t nseg = (h + max_rows - 1) / max_rows;
-            const int64_t want = spmm ? 1 : (int64_t)std::ceil(work_v / (double)o.tile_bytes);
-            return cut(std::max<int64_t>(nseg, std::min<int64_t>(want, (h + min_rows - 1) / min_rows)), false);
+            return cut(spmm ? (h + max_rows - 1) / max_rows : spmv_segments(o, h, work_v), false);
         };
         if (spmm && !mgroups.empty()) {
             // MFMA tiles (first launch): tall, multiples of 16 rows, only the
@@ -874,6 +885,7 @@ int build_host_plan_once(const SableVbr &v, const uint8_t *route, const SablePla
                 if (sv[s + 1] > sv[s]) emit(sv[s], sv[s + 1] - sv[s], true, false, 0);
         }
     }
+    if (survey) return SABLE_OK;
     // largest tiles first (LPT order for the persistent queue)
     std::vector<int32_t> order(P.tiles.size());
     std::iota(order.begin(), order.end(), 0);
