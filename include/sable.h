@@ -76,9 +76,11 @@ typedef struct {
     int32_t n_rhs;            /* SpMM RHS width N (multiple of 4); 1 for SpMV */
     int32_t wg;               /* workgroup size: 256 (default) */
     int32_t xcap;             /* max staged x columns per piece (16..4095) */
-    int64_t tile_bytes;       /* target algorithmic bytes per tile */
-    int32_t max_seg_rows;     /* upper bound on tile height (<= wg) */
-    int32_t min_seg_rows;     /* lower bound on tile height when splitting */
+    int64_t tile_bytes;       /* target algorithmic bytes per tile; in SpMM of the
+                                 MFMA tiles only (the others are cut into tasks) */
+    int32_t max_seg_rows;     /* upper bound on tile height (<= wg); MFMA tiles
+                                 have whole units of 16 rows */
+    int32_t min_seg_rows;     /* SpMV: lower bound on tile height when splitting */
     int32_t mode;             /* SABLE_MODE_*; -1 = default (grid) */
     int32_t grid;             /* persistent grid size; 0 = 8 per CU */
     int32_t unroll;           /* SpMV dense stream unroll (1,2,4,8); 0 = 4 */
@@ -88,10 +90,11 @@ typedef struct {
                                  (FP32-level, default); 2 = hi+lo, 3 passes */
     int32_t min_tiles;        /* tiles wanted at least: while a plan has fewer, its
                                  tile_bytes is halved (down to 16 KiB) so small
-                                 matrices still fill the device; 0 = 256 for
-                                 SpMM, and for SpMV a tile target (at most
-                                 tile_bytes) that follows the matrix and the
-                                 workgroups the device holds at once */
+                                 matrices still fill the device (in SpMM with
+                                 MFMA tiles); 0 = 256 for SpMM, and for SpMV a
+                                 tile target (at most tile_bytes) that follows
+                                 the matrix and the workgroups the device holds
+                                 at once */
     int32_t mfma_kchunk;      /* SpMM MFMA tiles: at most about this many 32-column
                                  k-steps per work item; a longer row tile is split
                                  along k into chunks whose partial sums a fixup

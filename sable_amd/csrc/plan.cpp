@@ -411,7 +411,8 @@ int64_t spmv_segments(const SablePlanOpts &o, int32_t h, double work)
 }
 
 // min_tiles asked for: the tile target is halved until there are that many
-// tiles (or tiles are 16 KiB).
+// tiles (or tiles are 16 KiB).  SpMM tiles without MFMA pieces do not follow
+// the target.
 int build_with_min_tiles(const SableVbr &v, const uint8_t *route, const SablePlanOpts &o, bool spans, HostPlan &P,
                          std::string &err)
 {
@@ -420,6 +421,7 @@ int build_with_min_tiles(const SableVbr &v, const uint8_t *route, const SablePla
         const int rc = build_host_plan_once(v, route, oo, spans, P, err);
         if (rc) return rc;
         if ((int64_t)P.tiles.size() >= oo.min_tiles || oo.tile_bytes <= 16 * 1024) return SABLE_OK;
+        if (o.op == SABLE_OP_SPMM && P.stats.ntiles_mfma == 0) return SABLE_OK;
         oo.tile_bytes = std::max<int64_t>(16 * 1024, oo.tile_bytes / 2);
     }
 }

@@ -3,11 +3,13 @@ more tiles than the device holds at once (768 workgroups of 512 threads), and
 what building a plan costs."""
 import subprocess
 import sys
+import time
 
 import numpy as np
 import pytest
 
 from conftest import ROOT
+from sable_amd import synth
 from sable_amd.runtime import Plan
 
 HEIGHT, WIDTH = 40, 400
@@ -54,3 +56,21 @@ def test_a_plan_is_held_once():
     out = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=120, check=True).stdout
     ntiles, times = out.split()
     assert int(ntiles) <= 768 and float(times) < 2.4
+
+
+def test_spmm_without_mfma_is_built_once():
+    """The tiles of such a plan do not follow tile_bytes: no number of tiles
+    asked for builds it again."""
+    vbr, _, _ = synth.mixed_vbr(4000, 60, 30, 120, 0.3, 0.5, (0.8, 1.0), (0.05, 0.3), seed=2)
+
+    def build(min_tiles):
+        best = []
+        for _ in range(3):
+            t = time.perf_counter()
+            plan = Plan.from_vbr(vbr, None, op="spmm", n_rhs=64, min_tiles=min_tiles, host_only=True)
+            best.append(time.perf_counter() - t)
+        return min(best), plan.export("tiles")
+
+    once, tiles = build(1)
+    asked, same = build(1 << 20)
+    assert np.array_equal(tiles, same) and asked < 2.5 * once
