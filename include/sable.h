@@ -118,7 +118,8 @@ typedef struct {
     int64_t rowptr_entries;   /* sparse index entries: CSR row pointers (SpMM) or
                                  row orders and wavefront tables (SpMV) */
     int64_t xmap_entries;     /* SpMV x staging map entries (x column per staged slot) */
-    int64_t descriptor_bytes; /* tiles + pieces + ranges */
+    int64_t descriptor_bytes; /* tiles + pieces + the staging map (SpMV); MFMA tiles + FP32
+                                 tasks + pieces + ranges (SpMM) */
     int64_t bytes_alg;        /* compulsory bytes of the executed format */
     int64_t flops_alg;        /* 2 * nnz * N */
     int64_t device_bytes;     /* device memory held by the plan */

@@ -491,8 +491,21 @@ int build_host_plan(const SableVbr &v, const uint8_t *route, const SablePlanOpts
                                        : build_for_slots(v, route, o, spans != 0, P, err);
         if (rc) return rc;
         const int64_t few = o.min_tiles > 0 ? o.min_tiles : SB_CUS;
-        if ((int64_t)P.tiles.size() >= few || !P.stats.nspans) return SABLE_OK;
+        if ((int64_t)P.tiles.size() >= few || !P.stats.nspans) break;
     }
+    SablePlanStats &S = P.stats;
+    const int32_t nm = S.ntiles_mfma;
+    if (P.op == SABLE_OP_SPMM && S.ntiles > nm)
+        P.tasks = f32_tasks(P.tiles, P.pieces, P.xr, P.tile_cost, nm, S.ntiles, P.n_rhs);
+    // what the kernels read: SpMV its tiles and the staging map, SpMM the MFMA
+    // tiles, the FP32 kernel's tasks and the ranges
+    const bool spmm = P.op == SABLE_OP_SPMM;
+    S.descriptor_bytes = (int64_t)((spmm ? nm : S.ntiles) * sizeof(SbTile) + P.pieces.size() * sizeof(SbPiece) +
+                                   P.tasks.size() * sizeof(SbTask)) +
+                         (spmm ? (int64_t)(P.xr.size() * sizeof(SbXRange)) : 4 * S.xmap_entries);
+    // a sparse entry: FP32 value and uint16 column (SpMV) or int32 X row
+    S.bytes_alg = 4 * S.dense_values + 4 * S.mfma_values + (spmm ? 8 : 6) * S.sparse_nnz + 4 * S.rowptr_entries +
+                  S.descriptor_bytes + 4LL * P.ncols * P.n_rhs + 4LL * P.nrows * P.n_rhs;
     return SABLE_OK;
 }
 
@@ -793,7 +806,7 @@ int build_host_plan_once(const SableVbr &v, const uint8_t *route, const SablePla
                         S.rowptr_entries += hs + 1;
                         push_xranges(P, sgroups[sr.group], pc);
                         P.pieces.push_back(pc);
-                        cost += 6.0 * tot + 4.0 * (hs + 1);
+                        cost += 8.0 * tot + 4.0 * (hs + 1);
                     }
                 } else {
                     cost += emit_wave_slices(P, S, t, sp, sgroups, hs, t.sp_waves ? t.sp_waves : nw, sp_glog);
@@ -915,11 +928,6 @@ int build_host_plan_once(const SableVbr &v, const uint8_t *route, const SablePla
     S.sparse_padded = (int64_t)P.sval.size();
     if (P.xmap.size() > (size_t)INT32_MAX) { err = "x staging map exceeds 2^31 entries"; return SABLE_ERR_UNSUPPORTED; }
     S.xmap_entries = (int64_t)P.xmap.size();
-    // what the kernels read: SpMV stages x through xmap, SpMM through the ranges
-    S.descriptor_bytes = (int64_t)(P.tiles.size() * sizeof(SbTile) + P.pieces.size() * sizeof(SbPiece)) +
-                         (spmm ? (int64_t)(P.xr.size() * sizeof(SbXRange)) : 4 * S.xmap_entries);
-    S.bytes_alg = 4 * S.dense_values + 4 * S.mfma_values + 6 * S.sparse_nnz + 4 * S.rowptr_entries +
-                  S.descriptor_bytes + 4LL * P.ncols * P.n_rhs + 4LL * P.nrows * P.n_rhs;
     S.flops_alg = 2 * S.nnz * (int64_t)P.n_rhs;
     S.scratch_bytes = P.part_blocks * 1024;
     S.wg = o.wg;
@@ -956,7 +964,7 @@ std::vector<SbTask> f32_tasks(const std::vector<SbTile> &tiles, const std::vecto
         }
         if (ti.rounds) waves += (int64_t)((tl.nrows + 31) / 32) * ((n_rhs + SB_F32_COLS - 1) / SB_F32_COLS);
         // the tile's sparse entries, from its cost estimate
-        ti.ent = std::max(0.0, (tile_cost[k] - 4.0 * tl.nrows * (double)ti.w - 2.0 * tl.nrows * n_rhs) / 6.0);
+        ti.ent = std::max(0.0, (tile_cost[k] - 4.0 * tl.nrows * (double)ti.w - 2.0 * tl.nrows * n_rhs) / 8.0);
     }
     const int wrows = waves < 2 * SB_SIMDS ? 16 : 32;
     std::vector<std::vector<Item>> per_tile;

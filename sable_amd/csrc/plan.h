@@ -20,10 +20,11 @@ struct HostPlan {
     std::vector<SbXRange> xr;
     std::vector<float> dval;      // FP32 dense pieces (both layouts)
     std::vector<float> sval;
-    std::vector<uint16_t> sidx;
+    std::vector<uint16_t> sidx;   // SpMM: on the host only (scol goes to the device)
     std::vector<int32_t> srowptr;
     std::vector<int32_t> scol;    // SpMM: X row of every entry of sval
     std::vector<int32_t> xmap;    // SpMV: x column per staged slot (-1 = zero pad)
+    std::vector<SbTask> tasks;    // SpMM: the FP32 kernel's task list
     std::vector<double> tile_cost;   // estimated bytes per tile (ordering)
     std::vector<int32_t> tile_phase; // 0: SpMM MFMA tile (first launch), 1: the rest
     int64_t part_blocks = 0;         // 1 KiB partial-sum blocks of the split MFMA tiles

@@ -537,11 +537,10 @@ int select_phases(const sable::HostPlan &h, const SablePlanOpts &o, int32_t ntil
 }
 
 // The task list of the FP32 SpMM phase, if there is one.
-int upload_tasks(const sable::HostPlan &h, std::vector<Phase> &phases, SbTask **d_tasks, int64_t &bytes)
+int upload_tasks(const std::vector<SbTask> &tasks, std::vector<Phase> &phases, SbTask **d_tasks, int64_t &bytes)
 {
     for (auto &ph : phases) {
         if (!ph.by_task()) continue;
-        const std::vector<SbTask> tasks = sable::f32_tasks(h.tiles, h.pieces, h.xr, h.tile_cost, ph.t0, ph.t1, h.n_rhs);
         if (tasks.size() > (size_t)INT32_MAX) return fail(SABLE_ERR_UNSUPPORTED, "the task list exceeds 2^31 entries");
         ph.ntasks = (int32_t)tasks.size();
         CHECKRC(upload(d_tasks, tasks, bytes));
@@ -834,7 +833,7 @@ int sable_plan_create(const SableVbr *vbr, const uint8_t *route, const SablePlan
     CHECKRC(upload(&p->d_xr, h.xr, bytes));
     CHECKRC(upload(&p->d_dval, h.dval, bytes));
     CHECKRC(upload(&p->d_sval, h.sval, bytes));
-    CHECKRC(upload(&p->d_sidx, h.sidx, bytes));
+    if (h.op == SABLE_OP_SPMV) CHECKRC(upload(&p->d_sidx, h.sidx, bytes));   // SpMM reads scol
     CHECKRC(upload(&p->d_srowptr, h.srowptr, bytes));
     CHECKRC(upload(&p->d_xmap, h.xmap, bytes));
     CHECKRC(upload(&p->d_scol, h.scol, bytes));
@@ -850,7 +849,7 @@ int sable_plan_create(const SableVbr *vbr, const uint8_t *route, const SablePlan
     HIPOK(hipStreamCreateWithFlags(&p->stream, hipStreamNonBlocking));
     p->own_stream = true;
     p->stats.rtc_used = 1;
-    CHECKRC(upload_tasks(h, p->phases, &p->d_tasks, bytes));
+    CHECKRC(upload_tasks(h.tasks, p->phases, &p->d_tasks, bytes));
     for (auto &ph : p->phases) {
         ph.grid = occupancy_grid(ph.rtc, ph.fn, ph.aot, ph.wg, std::max(1, ph.items()), o.grid);
         p->stats.rtc_used = p->stats.rtc_used && ph.rtc;
@@ -861,10 +860,11 @@ int sable_plan_create(const SableVbr *vbr, const uint8_t *route, const SablePlan
     // the big arrays live on the device now; keep only descriptors on the host
     p->host.dval = std::vector<float>();
     p->host.sval = std::vector<float>();
-    p->host.sidx = std::vector<uint16_t>();
+    if (h.op == SABLE_OP_SPMV) p->host.sidx = std::vector<uint16_t>();   // SpMM: kept for the export
     p->host.srowptr = std::vector<int32_t>();
     p->host.xmap = std::vector<int32_t>();
     p->host.scol = std::vector<int32_t>();
+    p->host.tasks = std::vector<SbTask>();
     p->keep_host = false;
     *out = p.release();
     return SABLE_OK;
@@ -928,7 +928,7 @@ int sable_plan_export(const SablePlan *p, int which, void *dst, int64_t *bytes)
     }
     *bytes = n;
     if (!dst || n == 0) return SABLE_OK;
-    if (p->keep_host || which <= 2) {
+    if (p->keep_host || which <= 2 || !dsrc) {
         std::memcpy(dst, hsrc, n);
     } else {
         HIPOK(hipMemcpy(dst, dsrc, n, hipMemcpyDeviceToHost));
@@ -1172,7 +1172,9 @@ int build_part(SablePlan *const *plans, const std::vector<int> &idx, const float
     for (size_t i = 0; i < order.size(); ++i) view.tile_cost[i] = cost[order[i]];
     for (int m : idx) view.ncols = std::max(view.ncols, plans[m]->host.ncols);
     CHECKRC(select_phases(view, p0->opts, nm, q.phases));
-    CHECKRC(upload_tasks(view, q.phases, &q.d_tasks, bytes));
+    if (q.op == SABLE_OP_SPMM)
+        view.tasks = sable::f32_tasks(view.tiles, view.pieces, view.xr, view.tile_cost, nm, q.ntiles, q.n_rhs);
+    CHECKRC(upload_tasks(view.tasks, q.phases, &q.d_tasks, bytes));
     for (auto &ph : q.phases)
         ph.grid = occupancy_grid(ph.rtc, ph.fn, ph.aot, ph.wg, std::max(1, ph.items()), grid);
     return SABLE_OK;
