@@ -159,7 +159,7 @@ int sable_plan_set_stream(SablePlan *plan, void *hip_stream);
 int sable_plan_export(const SablePlan *plan, int which, void *dst, int64_t *bytes);
 /* The kernel specialisation chosen for the plan (no reference counterpart):
  * spec6 = {kind, wg, unroll, xcap, nrhs, rtmax}, kind as in
- * sable_rtc_precompile. */
+ * sable_rtc_precompile (rtmax is no longer an option of any kernel). */
 int sable_plan_kernel_spec(const SablePlan *plan, int32_t *spec6);
 
 /* Replaces: one execution of the generated program's body,

@@ -57,7 +57,7 @@ def kernel_spec(plan_host):
 
 
 def _kernel_source(spec):
-    kind, wg, unroll, xcap, nrhs, rtmax = spec
+    kind, wg, unroll, xcap, nrhs = spec[:5]
     split = 2 if kind == KIND_SPMM_MFMA2 else 3
     body = {KIND_SPMV: "sb_spmv_body<SB_WG, SB_UNROLL, SB_XCAP>(a);",
             KIND_SPMM_F32: "sb_spmm_f32_body<SB_NRHS, SB_XCAP != 0>(a);",
@@ -68,7 +68,7 @@ def _kernel_source(spec):
               KIND_SPMM_F32: "SB_WG, SB_F32_MINWAVES"}.get(kind, "SB_WG, SB_MFMA_WAVES")
     return (f"// kernel specialisation for this matrix (compiled by hipRTC for gfx950)\n"
             f"#define SB_WG {wg}\n#define SB_UNROLL {unroll}\n#define SB_XCAP {xcap}\n"
-            f"#define SB_NRHS {nrhs}\n#define SB_RTMAX {rtmax}\n#define SB_SPLIT {split}\n"
+            f"#define SB_NRHS {nrhs}\n#define SB_SPLIT {split}\n"
             f"#include \"sable_kernels.h\"\n#include \"sable_mfma.h\"\n"
             f"extern \"C\" __global__ void __launch_bounds__({bounds}) sable_program({args} a)\n"
             f"{{ {body} }}\n")

@@ -8,9 +8,10 @@
 //    consecutive storage), so a row segment of that panel becomes one
 //    contiguous column-major sub-panel per column group;
 //  * sparse-routed blocks keep only their nonzeros (value != 0.0, the
-//    reference's routing count, utils/convert_real_to_vbr.py:41-47) as a CSR
-//    over the segment's rows with uint16 column indices into the group's x
-//    slice (entries of a row in ascending global column order);
+//    reference's routing count, utils/convert_real_to_vbr.py:41-47): in SpMV
+//    as wave slices with uint16 column indices into the group's x slice, in
+//    SpMM as a CSR over the segment's rows with the X row of every entry
+//    (entries of a row in ascending global column order);
 //  * MFMA-routed blocks (SpMM) are stored as FP32 in the exact register order
 //    of v_mfma_f32_16x16x32_bf16's A operand (16-row tile m, 32-column k-step
 //    s, lane l: A[16m + l%16][32s + 8(l/16) + j], j = 0..7).  A fragment

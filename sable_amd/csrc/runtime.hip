@@ -289,9 +289,9 @@ std::string spec_defines(const Spec &s)
 {
     char b[320];
     snprintf(b, sizeof b,
-             "#define SB_WG %d\n#define SB_UNROLL %d\n#define SB_XCAP %d\n#define SB_NRHS %d\n#define SB_RTMAX %d\n"
+             "#define SB_WG %d\n#define SB_UNROLL %d\n#define SB_XCAP %d\n#define SB_NRHS %d\n"
              "#define SB_SPLIT %d\n",
-             s.wg, s.unroll, s.xcap, s.nrhs, s.rtmax, s.split);
+             s.wg, s.unroll, s.xcap, s.nrhs, s.split);
     std::string d = b;
     if (const char *extra = getenv("SABLE_RTC_DEFINES")) {
         std::string e = extra;
@@ -344,7 +344,7 @@ struct Phase {
     int grid = 0;
     int wg = 256;       // workgroup size
     int32_t ntasks = 0; // FP32 SpMM: the phase's task list has this many places
-    int32_t spec[6] = {0, 0, 0, 0, 0, 0};   // kind, wg, unroll, xcap, nrhs, rtmax
+    int32_t spec[6] = {0, 0, 0, 0, 0, 0};   // kind, wg, unroll, xcap, nrhs; rtmax (no kernel's option)
     bool by_task() const { return spec[0] == 1; }   // FP32 SpMM: one workgroup per task
     // workgroups (work items) of the phase; MFMA: one per tile and column
     // group (the generic kernel takes all columns at once)

@@ -15,7 +15,8 @@ typedef unsigned long uint64_t;
 #endif
 
 #define SB_PIECE_DENSE 0        // column-major hs x ncols FP32 sub-panel
-#define SB_PIECE_SPARSE 1       // CSR over hs rows, uint16 local columns
+#define SB_PIECE_SPARSE 1       // SpMV: wave slices, uint16 columns of the staged x;
+                                // SpMM: CSR over hs rows, X rows in scol
 #define SB_PIECE_MFMA 2         // FP32 sub-panel in MFMA A-operand order (SpMM)
 
 // One unit of work: a row segment [row0, row0+nrows) of one block row of one
@@ -130,15 +131,16 @@ struct SbTask {
          ? 16 * ((WG) / 64) * SB_MFMA_UNITS(SB_MFMA_COLS(N, WG))    \
          : 256)
 
-// A panel piece of a tile: the tile's rows restricted to a group of blocks
-// whose columns (ncols <= the x staging capacity) are staged in LDS.
+// A panel piece of a tile: the tile's rows restricted to a group of blocks of
+// at most xcap columns together, which SpMV and the MFMA kernel stage in LDS.
 struct SbPiece {
     int64_t data_off;        // dense: float offset (multiple of 4) into dval
-                             // sparse: entry offset into sval/sidx
+                             // sparse: entry offset into sval and sidx (SpMV) or
+                             // scol (SpMM)
                              // mfma: float offset (multiple of 8) into dval
     int32_t kind;            // SB_PIECE_*
-    int32_t ncols;           // staged columns (x slice length)
-    int32_t xr_begin;        // staging ranges xr[xr_begin, xr_end)
+    int32_t ncols;           // columns (x slice length)
+    int32_t xr_begin;        // x ranges xr[xr_begin, xr_end)
     int32_t xr_end;
     int32_t rowptr_off;      // sparse, SpMM: CSR srowptr[rowptr_off .. +nrows] (relative
                              // to data_off); SpMV: per-wavefront {step offset,
@@ -156,7 +158,7 @@ struct SbPiece {
                              // extra rows zero, so a column's row quads are float4s)
 };
 
-// A contiguous run of x (or X rows) copied into the staging buffer.
+// A contiguous run of x (or X rows) that a piece's columns meet.
 struct SbXRange {
     int32_t col0;
     int32_t len;

@@ -9,7 +9,9 @@
 // block row; it owns those output rows and writes each exactly once, so no
 // atomics touch y/Y and results are deterministic.  A tile's pieces are the
 // column groups of its block row (dense FP32, dense FP32 in MFMA order, or
-// sparse CSR), each with an x slice of at most SB_XCAP columns staged in LDS.
+// sparse) of at most xcap columns each.  SpMV and the MFMA kernel stage a
+// piece's x slice or X rows in LDS; the FP32 SpMM kernel, whose tiles are cut
+// into tasks, reads X from memory into registers.
 #pragma once
 
 #include "sable_device.h"
