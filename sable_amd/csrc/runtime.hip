@@ -1230,7 +1230,12 @@ int sable_group_create(SablePlan *const *plans, int nplans, const float *const *
     }
     g->parts.resize(members.size());
     for (size_t j = 0; j < members.size(); ++j) {
-        const int rc = build_part(plans, members[j], x, y, mode, grid, g->parts[j]);
+        int rc;
+        try {
+            rc = build_part(plans, members[j], x, y, mode, grid, g->parts[j]);
+        } catch (const std::bad_alloc &) {
+            rc = fail(SABLE_ERR_OOM, "host allocation failed while building the group");
+        }
         if (rc) {
             for (auto &q : g->parts) free_part(q);
             return rc;
