@@ -94,7 +94,7 @@ typedef struct {
                                  MFMA tiles); 0 = 256 for SpMM, and for SpMV a
                                  tile target (at most tile_bytes) that follows
                                  the matrix and the workgroups the device holds
-                                 at once */
+                                 at once (1024 below 256 threads) */
     int32_t mfma_kchunk;      /* SpMM MFMA tiles: at most about this many 32-column
                                  k-steps per work item; a longer row tile is split
                                  along k into chunks whose partial sums a fixup

@@ -37,19 +37,22 @@ SablePlanOpts normalize_opts(const SablePlanOpts *in)
     if (o.op == SABLE_OP_SPMV) o.n_rhs = 1;
     if (o.wg <= 0) o.wg = 256;
     if (o.xcap <= 0) o.xcap = 4095;
-    // SpMV: 512 bytes per thread up to 256 threads.  A tile is as long as its
-    // round trips, so a batch ends with its longest tiles: 16 matrices of
-    // 2,000 to 32,000 rows, 122 MB, took 58 us with 512 KiB tiles of 256
-    // threads, 50 with 256 KiB, 37 with 128 KiB, 36 with 64 KiB; 64 matrices,
-    // 336 MB, 91, 72, 75 and 78 us.  With 128 threads 61 us from 256 KiB to
-    // 128 KiB, 45 with 64 KiB; with 64 threads 65 with 128 KiB, 37 with 32.
+    // SpMV members of a batch (min_tiles given): 512 bytes per thread up to 256
+    // threads.  A tile is as long as its round trips, so a batch ends with its
+    // longest tiles: 16 matrices of 2,000 to 32,000 rows, 122 MB, took 58 us
+    // with 512 KiB tiles of 256 threads, 50 with 256 KiB, 37 with 128 KiB, 36
+    // with 64 KiB; 64 matrices, 336 MB, 91, 72, 75 and 78 us.  With 128 threads
+    // 61 us from 256 KiB to 128 KiB, 45 with 64 KiB; with 64 threads 65 with
+    // 128 KiB, 37 with 32.  A plan on its own keeps 128 KiB: 20,000 rows of
+    // 10,000 stored columns took 186 us with 64 KiB tiles of 128 threads, 152
+    // with 512 KiB (a tile stages x for all its columns, however few its rows).
     // SpMM: MFMA tiles at N = 16 256 KiB (20,011 rows 31.2 -> 27.6 us, 50,000
     // rows 55.8 -> 54.3); at N = 32 half the tile took the 50,000 rows from
     // 65 to 72 us.
     if (o.tile_bytes <= 0)
-        o.tile_bytes = o.op == SABLE_OP_SPMV ? 512 * (int64_t)std::min(std::max(o.wg, 64), 256)
-                       : o.n_rhs <= 16              ? 256 * 1024
-                                                    : 512 * 1024;
+        o.tile_bytes = o.op == SABLE_OP_SPMM ? (o.n_rhs <= 16 ? 256 : 512) * 1024
+                       : o.min_tiles > 0     ? 512 * (int64_t)std::min(std::max(o.wg, 64), 256)
+                                             : 128 * 1024;
     if (o.max_seg_rows <= 0) o.max_seg_rows = o.wg;
     if (o.min_seg_rows <= 0) o.min_seg_rows = (o.op == SABLE_OP_SPMV) ? 8 : 16;
     if (o.mode < 0 || o.mode > 2) o.mode = SABLE_MODE_GRID;
@@ -57,8 +60,11 @@ SablePlanOpts normalize_opts(const SablePlanOpts *in)
     if (o.mfma_split != 2) o.mfma_split = 3;
     // SpMV tiles are light (stream-bound); SpMM tiles carry MFMA work and
     // gain from tall tiles (each staged X k-step serves every row)
-    // (0 for SpMV: the tile target follows the matrix, see build_host_plan)
-    if (o.min_tiles <= 0) o.min_tiles = (o.op == SABLE_OP_SPMV) ? 0 : 256;
+    // (0 for SpMV: the tile target follows the matrix, see build_host_plan;
+    // not below 256 threads, where its one round is of many small tiles: 40,000
+    // rows in block rows of 8, 64 threads, 62 us with 3,750 tiles and 43 with
+    // 1,250)
+    if (o.min_tiles <= 0) o.min_tiles = o.op == SABLE_OP_SPMM ? 256 : o.wg < 256 ? 1024 : 0;
     // k-split of MFMA row tiles only on request: on the 50k SpMM at N = 128
     // 32-k-step chunks measured 1-3.5 % slower than unsplit tiles (the fixup
     // launch and the partial-sum traffic outweigh the shorter chains)
@@ -428,7 +434,9 @@ int build_with_min_tiles(const SableVbr &v, const uint8_t *route, const SablePla
 }
 
 // SpMV on its own: tile_bytes bounds the tile target, which is set by the
-// workgroups the device holds at once (768 of 512 threads).  A tile costs
+// workgroups the device holds at once (768 of 512 threads; taken as two per
+// CU where it holds only one: 40,000 block rows of one row, unroll 8, 120 us
+// with tiles for 256 workgroups, 77 so, 88 halved until 1024).  A tile costs
 // several dependent round trips however small it is, so one round of tiles
 // that all fit is best where the block rows allow it; a second, nearly empty
 // round costs as much as the first.  The target is 1.4 times the bytes per
@@ -451,7 +459,7 @@ int build_for_slots(const SableVbr &v, const uint8_t *route, const SablePlanOpts
     Survey survey;
     const int rc = build_host_plan_once(v, route, o, spans, P, err, &survey);
     if (rc) return rc;
-    const int64_t slots = std::max<int64_t>(1, (int64_t)SB_SIMDS * std::max(2, SB_SPMV_WAVES(o.unroll)) * 64 / o.wg);
+    const int64_t slots = std::max<int64_t>(2 * SB_CUS, (int64_t)SB_SIMDS * std::max(2, SB_SPMV_WAVES(o.unroll)) * 64 / o.wg);
     const double share = (double)survey.bytes / (double)slots;
     auto with_target = [&](double bytes) {
         SablePlanOpts oo = o;

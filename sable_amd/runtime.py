@@ -161,10 +161,10 @@ class Plan:
         if tuned:
             from .autotune import tuned_options
             best = tuned_options(op, n_rhs)
-            if op == "spmv" and wg is not None and wg != best.get("wg"):
+            if op == "spmv" and wg is not None and wg != best.get("wg") and (min_tiles > 0 or wg == 256):
                 # measured for another workgroup size: 512 KiB tiles, right
                 # for 512 threads, are 64 round trips of 256 (the library's
-                # default follows the threads)
+                # default for a batch's members follows the threads)
                 best.pop("tile_bytes", None)
             for k, v in best.items():
                 if k in given and given[k] is None:
