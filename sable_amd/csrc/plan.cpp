@@ -815,7 +815,7 @@ int build_host_plan_once(const SableVbr &v, const uint8_t *route, const SablePla
                         S.rowptr_entries += hs + 1;
                         push_xranges(P, sgroups[sr.group], pc);
                         P.pieces.push_back(pc);
-                        cost += 8.0 * tot + 4.0 * (hs + 1);
+                        cost += 6.0 * tot + 4.0 * (hs + 1);
                     }
                 } else {
                     cost += emit_wave_slices(P, S, t, sp, sgroups, hs, t.sp_waves ? t.sp_waves : nw, sp_glog);
@@ -973,7 +973,7 @@ std::vector<SbTask> f32_tasks(const std::vector<SbTile> &tiles, const std::vecto
         }
         if (ti.rounds) waves += (int64_t)((tl.nrows + 31) / 32) * ((n_rhs + SB_F32_COLS - 1) / SB_F32_COLS);
         // the tile's sparse entries, from its cost estimate
-        ti.ent = std::max(0.0, (tile_cost[k] - 4.0 * tl.nrows * (double)ti.w - 2.0 * tl.nrows * n_rhs) / 8.0);
+        ti.ent = std::max(0.0, (tile_cost[k] - 4.0 * tl.nrows * (double)ti.w - 2.0 * tl.nrows * n_rhs) / 6.0);
     }
     const int wrows = waves < 2 * SB_SIMDS ? 16 : 32;
     std::vector<std::vector<Item>> per_tile;
