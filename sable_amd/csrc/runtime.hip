@@ -939,8 +939,8 @@ int sable_plan_export(const SablePlan *p, int which, void *dst, int64_t *bytes)
 // SpMV on host x and y of moderate size: x goes through pinned memory and a
 // copy kernel, and the SpMV kernel, which writes every y once and reads none,
 // writes it to pinned memory itself.  The runtime's copies of pageable memory
-// took 46 us a call for a 20,011-row matrix whose kernel takes 12; this way
-// takes 33.  Up to SABLE_PINNED_ROWS each the pinned memory is small (8 MiB).
+// took 47 us a call for a 20,011-row matrix whose kernel takes 7; this way
+// takes 29 (1,000,000 rows of 100 x 100 blocks 464 and 394).  Up to SABLE_PINNED_ROWS each the pinned memory is small (8 MiB).
 #define SABLE_PINNED_ROWS (1 << 20)
 
 static int run_host_spmv(SablePlan *p, const float *x, float *y, int64_t nx, int64_t ny, bool &taken)

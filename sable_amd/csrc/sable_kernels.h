@@ -271,7 +271,7 @@ __device__ __forceinline__ void sb_dense_piece(const SB_G sb_f4 *__restrict__ P,
     // batch is in flight per round trip.  A copy-free form (two buffers that
     // trade roles) keeps two in flight but needs about 113 VGPRs (4 waves
     // per SIMD, two 512-thread workgroups per CU) and measured no faster on
-    // the 100k matrix: the kernel runs at about 85 % of a cold streaming
+    // the 100k matrix: the kernel runs at about 90 % of a cold streaming
     // read of the same bytes either way.
     sb_f4 nxt[UNROLL];
     for (int b = 0; b < nbatch; ++b) {
@@ -517,11 +517,15 @@ __device__ __forceinline__ void sb_spmv_body(const SbSpmvArgs &a)
 // twice the vector ALUs' rate without packed instructions.  The vector
 // kernel this replaced (4 rows x 8 columns per thread, X staged in LDS) took
 // 260 us on the 50,000-row SpMM at N = 128 (35 M dense values, 0.9 M
-// entries) and 122 us on a 3,001-row one at N = 512; this one takes 175 and
-// 34 us.  On dense blocks alone it runs at 69 TFLOP/s (127 us): vector and
-// memory instructions take matrix time (both use the FP32 lanes and register
-// ports), and long tiles share SIMDs with others.  Measured slower, dense
-// blocks alone / with the entries: X staged through LDS (149 / 188 us),
+// entries) and 122 us on a 3,001-row one at N = 512; this one takes 173 and
+// 35 us.  Uniform tiles (256 block rows of 16 blocks of 128 x 128) run at
+// 113 TFLOP/s, the matrix units busy for 73 % of the launch, with 0.3 other
+// vector instructions and 0.25 loads per matrix instruction and the
+// wavefronts queued at the issue (72 % of their cycles).  On the 50,000-row
+// SpMM they are busy for 37 %: 1.9 other vector instructions (the entries'
+// products) and 0.45 loads per matrix instruction, 54 % of the wavefronts'
+// cycles waiting for loads.  Measured slower there, dense blocks alone / with
+// the entries, against 127 / 175 us: X staged through LDS (149 / 188 us),
 // 32-column tasks (155 / 213 us), one wavefront per workgroup without the
 // barrier (132 / 184 us).
 
